@@ -77,6 +77,10 @@ struct GemmArgs {
   // i-tiles per group of the grouped tile order (grouped_tile); 0: 8.  The
   // order only decides which workgroup computes which tile, never a result.
   int gi;
+  // pad: the operands are zero-padded copies (ragged.h), readable in whole
+  // chunks of 8 columns past I / J; sc: the output rows allow no 8-byte
+  // stores (J or ldc no multiple of 4, or c not 8-byte aligned)
+  int pad, sc;
 };
 
 // s * y + t * x as the Newton-Schulz combination steps take it (x is the
@@ -178,6 +182,9 @@ CONCORD_DEV void gemm_tile_of(const GemmArgs& g, int w, int& split, int& bi, int
 // returns CONCORD_OK, an error code, or -1 when the generic kernel must run
 int gemm_fast_launch(int mode, const GemmArgs& g, void* workspace, size_t ws_bytes,
                      hipStream_t st, const char* what);
+// whether gemm_fast_launch takes these operands (for WGRAD: with the
+// transpose-read kernel)
+bool gemm_fast_takes(int mode, const GemmArgs& g);
 // WGRAD whose epilogue also writes the v-hat partial sums of the bf16 output
 // (vhat_tile.h order) into vh_pr / vh_pc; -1 when the shape or its alignment
 // does not run the transpose-read kernel, or when the plan given split_room

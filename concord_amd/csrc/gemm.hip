@@ -21,6 +21,8 @@
 // fixup (the second finisher adds the first's fp32 partial: a + b = b + a).
 // Tiles are mapped XCD-aware: workgroup w runs on XCD w % 8, and each XCD
 // gets a compact block of the tile grid so its L2 serves shared operands.
+#include <algorithm>
+
 #include "gemm.h"
 #include "update_fast.h"
 #include "vhat.h"
@@ -435,10 +437,170 @@ static Plan plan_gemm(int64_t I, int64_t J, int64_t R, bool allow_split) {
   return best;
 }
 
+// ---- ragged operands ---------------------------------------------------------
+// The fast kernels move 16-byte chunks, so a layer whose N or K is no
+// multiple of 8 (a 65-word vocabulary head, 4-channel patch rows of 36) has
+// operands they cannot read.  Its products run on zero-padded copies in the
+// workspace: x and dy with rows of ceil8 columns, the weight decoded to bf16
+// rows of ceil8(K) with ceil8(N) rows.  The padding adds zero terms only, so
+// each output is the fp32 sum of the same products, and the outputs are
+// stored at their own ragged rows.  The copies are one pass over each operand;
+// the generic kernel instead gathers element by element in every tile, and
+// splits at most two ways.  Generic against copies (graph-timed, copies
+// included): 384 -> 65 at 16384 tokens, forward 76 -> 20 us, dgrad 209 -> 16,
+// wgrad 585 -> 25; 645 -> 2050 at 300 tokens 90 -> 24, 169 -> 23, 94 -> 21;
+// 400 -> 151 at 4 tokens 18.5 -> 10.8, 14.1 -> 12.3, 8.8 -> 7.4.
+// The copies cost up to two launches more, which the generic kernel beats
+// only where it has next to nothing to do (ragged_pays): a reduction of one
+// stage over few rows (forward 30 -> 1001 at 4 tokens 8.9 against 12.8 us,
+// 9 -> 9 at 200 tokens 12.0 against 13.1), or a layer of a few elements
+// (3 -> 5 at one token, backward 25 against 28 us).
+static bool ragged_pays(int64_t I, int64_t R) { return R > TR || I >= 512; }
+constexpr double kRaggedWork = 4096;   // M N K from which the copies are made at all
+
+static int64_t ceil8(int64_t v) { return (v + 7) / 8 * 8; }
+static size_t round256(size_t b) { return (b + 255) / 256 * 256; }
+
+// bytes of the padded copies of a layer's x, dy and weight (0: all of its
+// widths are multiples of 8, or the layer is tiny)
+struct RaggedRoom { size_t x, dy, w, total; };
+static RaggedRoom ragged_room(int64_t M, int64_t N, int64_t K) {
+  RaggedRoom r{0, 0, 0, 0};
+  if ((double)M * (double)N * (double)K < kRaggedWork || (N % 8 == 0 && K % 8 == 0)) return r;
+  r.x = round256((size_t)M * ceil8(K) * 2);
+  r.dy = round256((size_t)M * ceil8(N) * 2);
+  r.w = round256((size_t)ceil8(N) * ceil8(K) * 2);
+  r.total = r.x + r.dy + r.w;
+  return r;
+}
+
+// dst[r][c] = src[r][c] for r < rows and c < cols, 0 up to drows x dcols
+// (dcols a multiple of 8, dst 16-byte aligned).  PACKED: the source is packed
+// words, decoded as the materialised weight is.  One thread per 8 columns.
+template <bool PACKED>
+__global__ __launch_bounds__(256) void pad_rows_kernel(const void* __restrict__ src, int64_t ld, int64_t rows,
+                                                       int64_t cols, const int8_t* row_exp, const int8_t* col_exp,
+                                                       int32_t bias, uint16_t* __restrict__ dst, int64_t drows,
+                                                       int64_t dcols) {
+  const int64_t cpr = dcols / 8, total = drows * cpr;
+  for (int64_t q = (int64_t)blockIdx.x * 256 + threadIdx.x; q < total; q += (int64_t)gridDim.x * 256) {
+    const int64_t r = q / cpr, c = (q % cpr) * 8;
+    uint32_t w[4] = {0, 0, 0, 0};
+    if (r < rows) {
+      const int32_t te = PACKED ? (int32_t)row_exp[r] - bias : 0;
+#pragma unroll
+      for (int e = 0; e < 8; ++e) {
+        if (c + e >= cols) break;
+        uint32_t h;
+        if (PACKED)
+          h = pack_bf16x2(decode_word(((const int32_t*)src)[r * ld + c + e], te + (int32_t)col_exp[c + e]), 0.0f) & 0xFFFFu;
+        else
+          h = ((const uint16_t*)src)[r * ld + c + e];
+        w[e / 2] |= h << (16 * (e & 1));
+      }
+    }
+    *reinterpret_cast<uint4*>(dst + r * dcols + c) = make_uint4(w[0], w[1], w[2], w[3]);
+  }
+}
+
+static void pad_rows_launch(bool packed, const void* src, int64_t ld, int64_t rows, int64_t cols,
+                            const int8_t* row_exp, const int8_t* col_exp, int32_t bias, uint16_t* dst, int64_t drows,
+                            hipStream_t st) {
+  const int64_t dcols = ceil8(cols), blocks = std::min<int64_t>(cdiv(drows * (dcols / 8), 256), 4096);
+  if (packed)
+    hipLaunchKernelGGL(pad_rows_kernel<true>, dim3((unsigned)blocks), dim3(256), 0, st, src, ld, rows, cols, row_exp,
+                       col_exp, bias, dst, drows, dcols);
+  else
+    hipLaunchKernelGGL(pad_rows_kernel<false>, dim3((unsigned)blocks), dim3(256), 0, st, src, ld, rows, cols, nullptr,
+                       nullptr, 0, dst, drows, dcols);
+}
+
+// The padded operands of one call, made on first use at the workspace's end
+// (`inner` bytes before them stay for the products' split-K partials).
+struct Ragged {
+  char* base = nullptr;
+  size_t inner = 0;
+  RaggedRoom room{0, 0, 0, 0};
+  hipStream_t st;
+  // false: the shape is not ragged, or the workspace has no room
+  bool init(int64_t M, int64_t N, int64_t K, void* workspace, size_t ws_bytes, hipStream_t stream) {
+    room = ragged_room(M, N, K);
+    st = stream;
+    if (room.total == 0 || !workspace || ws_bytes < kSplitkCounterBytes + room.total + 256) return false;
+    inner = (ws_bytes - room.total) / 256 * 256;
+    base = (char*)workspace + inner;
+    return true;
+  }
+  static bool plain(const uint16_t* p, int64_t ld, int64_t cols) {
+    return cols % 8 == 0 && ld % 8 == 0 && ((uintptr_t)p % 16) == 0;
+  }
+  // (p, ld) of an activation operand, replaced by a padded copy where needed
+  void activation(const uint16_t*& p, int64_t& ld, int64_t rows, int64_t cols, size_t off) const {
+    if (plain(p, ld, cols)) return;
+    uint16_t* d = (uint16_t*)(base + off);
+    pad_rows_launch(false, p, ld, rows, cols, nullptr, nullptr, 0, d, rows, st);
+    p = d;
+    ld = ceil8(cols);
+  }
+  void x(const uint16_t*& p, int64_t& ld, int64_t M, int64_t K) const { activation(p, ld, M, K, 0); }
+  void dy(const uint16_t*& p, int64_t& ld, int64_t M, int64_t N) const { activation(p, ld, M, N, room.x); }
+  // the weight operand of g (packed words, or bf16 rows) as padded bf16 rows
+  const uint16_t* weight(const GemmArgs& g, bool packed, int64_t N, int64_t K) const {
+    uint16_t* d = (uint16_t*)(base + room.x + room.dy);
+    pad_rows_launch(packed, g.b, g.ldb, N, K, g.row_exp, g.col_exp, g.bias, d, ceil8(N), st);
+    return d;
+  }
+};
+
+static bool ragged_out(const GemmArgs& g) { return g.ldc % 4 != 0 || g.J % 4 != 0 || ((uintptr_t)g.c % 8) != 0; }
+
+// forward or dgrad of a ragged layer on its padded operands; -1 where the
+// fast kernels do not take them either
+template <int MODE>
+static int ragged_product(const Ragged& rg, const GemmArgs& g, void* workspace, const char* what) {
+  constexpr bool FWD = MODE == MODE_FWD || MODE == MODE_FWD_BF16;
+  GemmArgs p = g;
+  const int64_t M = g.I, N = FWD ? g.J : g.R, K = FWD ? g.R : g.J;
+  if (FWD) rg.x(p.a, p.lda, M, K);
+  else rg.dy(p.a, p.lda, M, N);
+  p.b = rg.weight(g, MODE == MODE_FWD || MODE == MODE_DGRAD, N, K);
+  p.ldb = ceil8(K);
+  p.R = ceil8(g.R);
+  p.row_exp = p.col_exp = nullptr;
+  p.pad = 1;
+  p.sc = ragged_out(g);
+  return gemm_fast_launch(FWD ? MODE_FWD_BF16 : MODE_DGRAD_BF16, p, workspace, rg.inner, rg.st, what);
+}
+
+// g (a WGRAD) on padded dy and x
+static void ragged_wgrad(const Ragged& rg, GemmArgs& g) {
+  const uint16_t* x = (const uint16_t*)g.b;
+  rg.dy(g.a, g.lda, g.R, g.I);
+  rg.x(x, g.ldb, g.R, g.J);
+  g.b = x;
+  g.pad = 1;
+  g.sc = ragged_out(g);
+}
+
 template <int MODE>
 static int launch_gemm(GemmArgs g, void* workspace, size_t ws_bytes, hipStream_t st,
                        const char* what) {
   if (g.I == 0 || g.J == 0) return CONCORD_OK;
+  if (!gemm_fast_takes(MODE, g)) {
+    constexpr bool FWD = MODE == MODE_FWD || MODE == MODE_FWD_BF16;
+    Ragged rg;
+    if (MODE == MODE_WGRAD) {
+      if (rg.init(g.R, g.I, g.J, workspace, ws_bytes, st)) {
+        GemmArgs p = g;
+        ragged_wgrad(rg, p);
+        const int rc = gemm_fast_launch(MODE, p, workspace, rg.inner, st, what);
+        if (rc != -1) return rc;
+      }
+    } else if (!g.ay && ragged_pays(g.I, g.R) && rg.init(g.I, FWD ? g.J : g.R, FWD ? g.R : g.J, workspace, ws_bytes, st)) {
+      const int rc = ragged_product<MODE>(rg, g, workspace, what);
+      if (rc != -1) return rc;
+    }
+  }
   const int fast = gemm_fast_launch(MODE, g, workspace, ws_bytes, st, what);
   if (fast != -1) return fast;
   const bool can_split = workspace != nullptr;
@@ -533,7 +695,14 @@ extern "C" size_t concord_gemm_workspace_bytes(int64_t M, int64_t N, int64_t K) 
   if (K < 1) K = 1;
   const size_t a = splitk_partials(MODE_FWD, M, N, K), b = splitk_partials(MODE_DGRAD, M, K, N),
                c = splitk_partials(MODE_WGRAD, N, K, M);
-  const size_t m = a > b ? (a > c ? a : c) : (b > c ? b : c);
+  size_t m = a > b ? (a > c ? a : c) : (b > c ? b : c);
+  const RaggedRoom r = ragged_room(M, N, K);
+  if (r.total) {   // the padded operands, and the partials of the products on them
+    const int64_t N8 = ceil8(N), K8 = ceil8(K);
+    for (size_t v : {splitk_partials(MODE_FWD_BF16, M, N, K8), splitk_partials(MODE_DGRAD_BF16, M, K, N8)})
+      if (v > m) m = v;
+    m = round256(m) + r.total + 256;
+  }
   return kSplitkCounterBytes + ((m + 255) / 256) * 256;
 }
 
@@ -611,6 +780,24 @@ static int wgrad_vhat_impl(const GemmArgs* gd, const uint16_t* dy, int64_t ld_dy
   int rc = -1;
   GemmArgs pend;        // a dgrad split-K reduction the finalize launch carries
   int pend_rbi = 0;
+  Ragged rg;
+  GemmArgs gdr;
+  if (!gemm_fast_takes(MODE_WGRAD, g) && rg.init(M, N, K, gemm_workspace, gemm_workspace_bytes, st)) {
+    // dy and x padded once, for both products
+    ragged_wgrad(rg, g);
+    if (gd && gd->I > 0 && gd->J > 0) {
+      gdr = *gd;
+      gdr.a = g.a;
+      gdr.lda = g.lda;
+      if (!gemm_fast_takes(MODE_DGRAD, gdr) && ragged_pays(gd->I, gd->R))
+        rc = ragged_product<MODE_DGRAD>(rg, gdr, gemm_workspace, what);
+      if (rc == -1) rc = launch_gemm<MODE_DGRAD>(gdr, gemm_workspace, rg.inner, st, what);
+      if (rc != CONCORD_OK) return rc;
+      rc = -1;
+    }
+    gemm_workspace_bytes = rg.inner;
+    gd = nullptr;
+  }
   if (gd && gd->I > 0 && gd->J > 0) {
     rc = gemm_dgrad_wgrad_vhat_launch(*gd, gemm_workspace, gemm_workspace ? gemm_workspace_bytes : 0, g, st,
                                       what, &tiles_j, &pend, &pend_rbi);
@@ -627,6 +814,7 @@ static int wgrad_vhat_impl(const GemmArgs* gd, const uint16_t* dy, int64_t ld_dy
   if (rc == -1) rc = gemm_wgrad_vhat_split_launch(g, gemm_workspace, gemm_workspace_bytes, st, what, &tiles_j);
   if (rc == -1) {   // unaligned WGRAD: the plain product, then the partials kernels
     g.bpart = nullptr;
+    g.vh_pr = g.vh_pc = nullptr;
     rc = launch_gemm<MODE_WGRAD>(g, gemm_workspace, gemm_workspace_bytes, st, what);
     if (rc != CONCORD_OK) return rc;
     vhat_partials_launch(grad_w, ld_gw, N, K, pr, pc, st);

@@ -317,7 +317,8 @@ struct ColsBf16 {
   CONCORD_DEV void init(const uint16_t* band, int64_t ld, int64_t cols_left, int64_t R, int t) {
     rb = G::rb(t);
     ld2 = (uint32_t)(ld * 2);
-    rs = make_rsrc(band, nrec(((R - 1) * ld + cols_left) * 2));
+    // (cols_left is a multiple of 4, or the operand is padded to one)
+    rs = make_rsrc(band, nrec(((R - 1) * ld + (cols_left + 3) / 4 * 4) * 2));
 #pragma unroll
     for (int q = 0; q < PER; ++q) {
       const int64_t col = G::col(t, q);
@@ -464,6 +465,33 @@ CONCORD_DEV float* partial_slot(const GemmArgs& g, int tile, int split, int aw) 
   return g.part + ((int64_t)tile * g.splits + split) * ((int64_t)NAW * NI * NJ * 256) + (int64_t)aw * NI * NJ * 256;
 }
 
+// the bias of columns j .. j + 3 (j < J)
+CONCORD_DEV void load_bias4(const GemmArgs& g, int64_t j, float (&bs)[4]) {
+  if (g.sc) {
+#pragma unroll
+    for (int e = 0; e < 4; ++e) bs[e] = j + e < g.J ? bf16_to_f32(g.vbias[j + e]) : 0.f;
+    return;
+  }
+  const uint2 b4 = *reinterpret_cast<const uint2*>(g.vbias + j);
+  bs[0] = __uint_as_float(b4.x << 16);
+  bs[1] = __uint_as_float(b4.x & 0xFFFF0000u);
+  bs[2] = __uint_as_float(b4.y << 16);
+  bs[3] = __uint_as_float(b4.y & 0xFFFF0000u);
+}
+
+// 4 bf16 (o) to columns j .. j + 3 of an output row (j < J)
+CONCORD_DEV void store4(const GemmArgs& g, int64_t i, int64_t j, uint2 o) {
+  uint16_t* c = g.c + i * g.ldc + j;
+  if (!g.sc) {
+    *reinterpret_cast<uint2*>(c) = o;
+    return;
+  }
+  const uint32_t w[2] = {o.x, o.y};
+#pragma unroll
+  for (int e = 0; e < 4; ++e)
+    if (j + e < g.J) c[e] = (uint16_t)(w[e / 2] >> (16 * (e & 1)));
+}
+
 template <int MODE, int NI, int NJ, int BI, int BJ, int NAW>
 CONCORD_DEV void epilogue(const GemmArgs& g, f32x4 (&acc)[NI][NJ], int64_t i0, int64_t j0, int ra, int rb,
                           int split, int tile, int aw, int t, int nthreads, uint16_t* stage) {
@@ -495,13 +523,7 @@ CONCORD_DEV void epilogue(const GemmArgs& g, f32x4 (&acc)[NI][NJ], int64_t i0, i
 #pragma unroll
           for (int e = 0; e < 4; ++e) sc[e] = exp2i(sbyte(e4, e) - g.bias);
         }
-        if (g.vbias) {
-          const uint2 b4 = *reinterpret_cast<const uint2*>(g.vbias + j);
-          bs[0] = __uint_as_float(b4.x << 16);
-          bs[1] = __uint_as_float(b4.x & 0xFFFF0000u);
-          bs[2] = __uint_as_float(b4.y << 16);
-          bs[3] = __uint_as_float(b4.y & 0xFFFF0000u);
-        }
+        if (g.vbias) load_bias4(g, j, bs);
       }
 #pragma unroll
       for (int x = 0; x < NI; ++x) {
@@ -518,7 +540,14 @@ CONCORD_DEV void epilogue(const GemmArgs& g, f32x4 (&acc)[NI][NJ], int64_t i0, i
   // row-contiguous stores: 8 bf16 (16 bytes) per thread when the output
   // allows, else 4 (J % 4 == 0, ldc % 4 == 0, 8-byte aligned base)
   const bool v16 = (g.ldc % 8 == 0) && (g.J % 8 == 0) && (((uintptr_t)g.c % 16) == 0);
-  if (g.sym) {
+  if (g.sc) {
+    // ragged rows: one element per thread, consecutive threads consecutive columns
+    for (int c = t; c < BI * BJ; c += nthreads) {
+      const int rl = c / BJ, cl = c % BJ;
+      const int64_t i = i0 + rl, j = j0 + cl;
+      if (i < g.I && j < g.J) g.c[i * g.ldc + j] = stage[rl * LDO + cl];
+    }
+  } else if (g.sym) {
     // symmetric product: each element (i, j) with i <= j goes to (i, j) and
     // (j, i); the tile's elements below the diagonal are left to the tile
     // holding their mirror image (every element is written once)
@@ -605,13 +634,7 @@ CONCORD_DEV void splitk_reduce_item_sp(const GemmArgs& g, int64_t idx) {
 #pragma unroll
     for (int e = 0; e < 4; ++e) sc[e] = exp2i(sbyte(e4, e) - g.bias);
   }
-  if (g.vbias) {
-    const uint2 b4 = *reinterpret_cast<const uint2*>(g.vbias + j);
-    bs[0] = __uint_as_float(b4.x << 16);
-    bs[1] = __uint_as_float(b4.x & 0xFFFF0000u);
-    bs[2] = __uint_as_float(b4.y << 16);
-    bs[3] = __uint_as_float(b4.y & 0xFFFF0000u);
-  }
+  if (g.vbias) load_bias4(g, j, bs);
   float v[4];
 #pragma unroll
   for (int e = 0; e < 4; ++e) v[e] = __fadd_rn(__fmul_rn(sum[e], sc[e]), bs[e]);
@@ -636,7 +659,7 @@ CONCORD_DEV void splitk_reduce_item_sp(const GemmArgs& g, int64_t idx) {
     }
     return;
   }
-  *reinterpret_cast<uint2*>(g.c + i * g.ldc + j) = o;
+  store4(g, i, j, o);
 }
 
 // splitk_reduce_item_sp for the launch's split count (uniform), 2 .. kGemmMaxSplits
@@ -750,7 +773,7 @@ struct ReduceVh {
 #pragma unroll
         for (int e = 0; e < 4; ++e) s_g2[((x * NJ + y) * 4 + e) * 64 + lane] = __fmul_rn(v[e], v[e]);
         const int64_t i = row0 + x * 16 + (lane & 15), j = col0 + y * 16 + 4 * (lane >> 4);
-        if (i < g.I && j < g.J) *reinterpret_cast<uint2*>(g.c + i * g.ldc + j) = make_uint2(lo, hi);
+        if (i < g.I && j < g.J) store4(g, i, j, make_uint2(lo, hi));
       }
     }
     if (x == 1 && g.bpart && aw % WJ == 0) {
@@ -1421,7 +1444,8 @@ struct TrDma {
     ld2 = ld * 2;
     lrow = lane / (ROWB / 16);
     const uint64_t base = (uint64_t)(uintptr_t)band;
-    const int64_t bytes = ((R - 1) * ld + (cols_left < COLS ? cols_left : COLS)) * 2;
+    // (cols_left is a multiple of 8, or the operand is padded to one)
+    const int64_t bytes = ((R - 1) * ld + (cols_left < COLS ? (cols_left + 7) / 8 * 8 : COLS)) * 2;
     rs = i32x4{(int32_t)(uint32_t)base, (int32_t)(uint32_t)((base >> 32) & 0xFFFF), (int32_t)nrec(bytes),
                0x00020000};
     for (int e = 0; e < 4; ++e) rs[e] = __builtin_amdgcn_readfirstlane(rs[e]);
@@ -1790,7 +1814,8 @@ struct TrRowsB {
     col = 4 * (t % CG);
     rg = t / CG;
     ldb = (uint32_t)(ld * ES);
-    rs = make_rsrc(band, nrec(((R - 1) * ld + cols_left) * ES));
+    // (cols_left is a multiple of 4, or the operand is padded to one)
+    rs = make_rsrc(band, nrec(((R - 1) * ld + (cols_left + 3) / 4 * 4) * ES));
     if (PACKED) es = make_rsrc(exps, (uint32_t)R);
     voff = col < cols_left ? (uint32_t)((8 * rg * ld + col) * ES) : kOOB;
   }
@@ -2130,10 +2155,14 @@ static bool fits31(int64_t bytes) { return bytes < ((int64_t)1 << 30); }
 
 // alignment and extent rules of the fast kernels, per mode
 static bool eligible(int mode, const GemmArgs& g) {
-  if (!(g.ldc % 4 == 0 && g.J % 4 == 0 && al(g.c, 8))) return false;
+  // the bf16 kernels store any output row; the combine, the packed modes'
+  // exponent loads and the symmetric store take whole 4-column groups
+  const bool out4 = g.ldc % 4 == 0 && g.J % 4 == 0 && al(g.c, 8);
+  if (!out4 && !g.sc) return false;
+  if (g.sc && (g.ay || mode == MODE_FWD || mode == MODE_DGRAD)) return false;
   // the combine operand is read at the output's positions, 16 bytes at a time
   if (g.ay && !(g.ldy % 8 == 0 && g.ldc % 8 == 0 && g.J % 8 == 0 && al(g.ay, 16) && al(g.c, 16))) return false;
-  if (g.vbias && !al(g.vbias, 8)) return false;
+  if (g.vbias && !g.sc && !al(g.vbias, 8)) return false;
   switch (mode) {
     case MODE_FWD:
       return g.lda % 8 == 0 && g.R % 8 == 0 && al(g.a, 16) && g.ldb % 4 == 0 && al(g.b, 16) &&
@@ -2150,7 +2179,7 @@ static bool eligible(int mode, const GemmArgs& g) {
       return g.lda % 8 == 0 && g.R % 8 == 0 && al(g.a, 16) && g.ldb % 4 == 0 && al(g.b, 8) &&
              fits31(((g.I - 1) * g.lda + g.R) * 2) && fits31(((g.R - 1) * g.ldb + g.J) * 2);
     case MODE_WGRAD:
-      return g.lda % 4 == 0 && g.I % 4 == 0 && al(g.a, 8) && g.ldb % 4 == 0 && al(g.b, 8) &&
+      return g.lda % 4 == 0 && (g.pad || g.I % 4 == 0) && al(g.a, 8) && g.ldb % 4 == 0 && al(g.b, 8) &&
              fits31(((g.R - 1) * g.lda + g.I) * 2) && fits31(((g.R - 1) * g.ldb + g.J) * 2);
   }
   return false;
@@ -2158,7 +2187,8 @@ static bool eligible(int mode, const GemmArgs& g) {
 
 // the transpose-read WGRAD kernel moves 16-byte chunks of both operands
 static bool tr_eligible(const GemmArgs& g) {
-  return g.lda % 8 == 0 && g.I % 8 == 0 && al(g.a, 16) && g.ldb % 8 == 0 && g.J % 8 == 0 && al(g.b, 16);
+  return g.lda % 8 == 0 && al(g.a, 16) && g.ldb % 8 == 0 && al(g.b, 16) &&
+         (g.pad || (g.I % 8 == 0 && g.J % 8 == 0));
 }
 
 // split-K: sum the partials once every split has stored them
@@ -2290,6 +2320,10 @@ size_t gemm_fast_partial_bytes(int mode, int64_t I, int64_t J, int64_t R) {
 }
 
 int64_t gemm_wgrad_vhat_tiles_j(int64_t J) { return cdiv(J, 128); }
+
+bool gemm_fast_takes(int mode, const GemmArgs& g) {
+  return eligible(mode, g) && (mode != MODE_WGRAD || tr_eligible(g));
+}
 
 int gemm_wgrad_vhat_launch(const GemmArgs& g0, size_t split_room, hipStream_t st, const char* what,
                            int* tiles_j) {

@@ -1,0 +1,118 @@
+"""Layers whose widths are no multiples of 8: the products run on zero-padded
+copies in the workspace (ragged operands, csrc/gemm.hip)."""
+import numpy as np
+import pytest
+import torch
+
+from gpu_util import DEV, dev, host, rand_state, sync
+
+pytestmark = pytest.mark.gpu
+
+# (M, N, K): the edges of the 8-column chunks and of the rule that makes the
+# copies (more than 64 terms, 512 rows, 4096 elements of work), one row or
+# column, a vocabulary head, 4-channel patch rows, odd widths past a tile
+SHAPES = [(1, 5, 3), (4, 32, 31), (4, 33, 31), (511, 65, 40), (511, 30, 64), (511, 30, 66), (512, 30, 64),
+          (512, 65, 384), (64, 9, 1001), (300, 2050, 645), (513, 1, 36), (1030, 4, 2880), (700, 129, 7), (600, 8, 9), (777, 100, 770),
+          (2050, 320, 36), (640, 257, 131), (520, 36, 1)]
+
+
+def _bound(exact, terms):
+    """One fp32 sum of the terms in any order (at most 2^14 of them, each
+    rounded at 2^-24 of the running sum of magnitudes) rounded once to bf16."""
+    return 2.0 ** -8 * np.abs(exact) + 2.0 ** -10 * 1e-2 * terms + 1e-30
+
+
+def _f64(t):
+    return t.detach().double().cpu().numpy()
+
+
+@pytest.mark.parametrize("M,N,K", SHAPES)
+def test_ragged_products_match_float64(oracle, M, N, K):
+    from concord_amd import packed_b as pb
+    rng = np.random.default_rng(M + 3 * N + 7 * K)
+    packed, re, ce = rand_state(rng, N, K, exp=(-2, 2), col=(-2, 2))
+    pk, red, ced = dev(packed), dev(re), dev(ce)
+    gen = torch.Generator().manual_seed(M)
+    x = torch.randn(M, K, generator=gen).to(torch.bfloat16).to(DEV)
+    dy = torch.randn(M, N, generator=gen).to(torch.bfloat16).to(DEV)
+    b = torch.randn(N, generator=gen).to(torch.bfloat16).to(DEV)
+    W = oracle.bf16_bits_to_f32(oracle.materialize(packed, re, ce)).astype(np.float64)
+    Wb = torch.from_numpy(W).to(torch.bfloat16).to(DEV)
+    xd, dyd, bd = _f64(x), _f64(dy), _f64(b)
+    y_ref, y_terms = xd @ W.T + bd, np.abs(xd) @ np.abs(W).T + np.abs(bd)
+    dx_ref, dx_terms = dyd @ W, np.abs(dyd) @ np.abs(W)
+    gw_ref, gw_terms = dyd.T @ xd, np.abs(dyd).T @ np.abs(xd)
+    for wbuf in (None, Wb):
+        y = pb._gemm_fwd(x, pk, red, ced, 15, b, wbuf)
+        dx = pb._gemm_dgrad(dy, pk, red, ced, 15, wbuf)
+        assert (np.abs(_f64(y) - y_ref) <= _bound(y_ref, y_terms)).all()
+        assert (np.abs(_f64(dx) - dx_ref) <= _bound(dx_ref, dx_terms)).all()
+    gw = pb._wgrad(dy, x)
+    sync()
+    assert (np.abs(_f64(gw) - gw_ref) <= _bound(gw_ref, gw_terms)).all()
+
+
+@pytest.mark.parametrize("M,N,K", SHAPES)
+def test_ragged_backward_entry_matches_separate_calls(oracle, M, N, K):
+    """The combined entry, the v-hat entry and the plain product agree bit for
+    bit on dx, grad_W and v-hat; the bias gradient matches the float64 sum."""
+    from concord_amd import packed_b as pb
+    rng = np.random.default_rng(M + N + K)
+    packed, re, ce = rand_state(rng, N, K, exp=(-3, 3), col=(-1, 1))
+    pk, red, ced = dev(packed), dev(re), dev(ce)
+    gen = torch.Generator().manual_seed(K)
+    x = torch.randn(M, K, generator=gen).to(torch.bfloat16).to(DEV)
+    dy = (torch.randn(M, N, generator=gen) * 1e-2).to(torch.bfloat16).to(DEV)
+    outs, gbs = [], []
+    for combined in (True, False):
+        vr, vc = torch.full((N,), 1e-4, device=DEV), torch.full((K,), 2e-4, device=DEV)
+        svi = torch.ones(1, device=DEV)
+        rm = torch.full((N,), 77, dtype=torch.int32, device=DEV)
+        cm = torch.full((K,), 88, dtype=torch.int32, device=DEV)
+        salt = torch.full((1,), 5, dtype=torch.int32, device=DEV)
+        args = (vr, vc, svi, 0.999, rm, cm, salt)
+        if combined:
+            dx, gw, gb = pb._dgrad_wgrad_vhat(dy, x, pk, red, ced, 15, *args, with_bias=True)
+        else:
+            dx = pb._gemm_dgrad(dy, pk, red, ced, 15, None)
+            gw, gb = pb._wgrad_vhat(dy, x, *args, with_bias=True)
+        sync()
+        outs.append([host(t) for t in (dx, gw, vr, vc, svi, rm, cm, salt)])
+        gbs.append(_f64(gb))
+    outs[1][1:2] = [host(pb._wgrad(dy, x))]
+    for a, b in zip(*outs):
+        np.testing.assert_array_equal(a, b)
+    vr, vc = np.full(N, 1e-4, np.float32), np.full(K, 2e-4, np.float32)
+    oracle.vhat_ema(outs[0][1], vr, vc, 0.999)
+    np.testing.assert_array_equal(outs[0][2], vr)
+    np.testing.assert_array_equal(outs[0][3], vc)
+    gb_ref, terms = _f64(dy).sum(0), np.abs(_f64(dy)).sum(0)
+    for gb in gbs:
+        assert (np.abs(gb - gb_ref) <= _bound(gb_ref, terms)).all()
+
+
+@pytest.mark.parametrize("M,N,K", [(600, 65, 40), (900, 30, 33)])
+def test_ragged_strided_and_small_workspace(oracle, M, N, K):
+    """Operands with their own row strides and unaligned bases, and a
+    workspace without room for the copies (the generic kernel), give the
+    products of the plain call."""
+    from concord_amd import _lib as C, packed_b as pb
+    rng = np.random.default_rng(N)
+    packed, re, ce = rand_state(rng, N, K, exp=(-2, 2), col=(-1, 1))
+    pk, red, ced = dev(packed), dev(re), dev(ce)
+    x = torch.randn(M, K, device=DEV).to(torch.bfloat16)
+    base = pb._gemm_fwd(x, pk, red, ced, 15, None, None).double()
+    xs = torch.zeros(M, K + 5, dtype=torch.bfloat16, device=DEV)
+    xs[:, 1:K + 1] = x
+    view = xs[:, 1:K + 1]
+    need = int(C.lib().concord_gemm_workspace_bytes(M, N, K))
+    for nbytes in (need, 16384):
+        ws = torch.zeros(nbytes, dtype=torch.uint8, device=DEV)
+        y = torch.full((M, N + 3), 7.0, dtype=torch.bfloat16, device=DEV)
+        C.check(C.lib().concord_dqgemm_fwd(C.ptr(view), view.stride(0), C.ptr(pk), pk.stride(0), C.ptr(red), C.ptr(ced),
+                                           15, None, C.ptr(y), y.stride(0), M, N, K, C.ptr(ws), nbytes,
+                                           C.stream_of(torch.device(DEV))), "fwd")
+        sync()
+        assert (y[:, N:] == 7.0).all()
+        err = (y[:, :N].double() - base).norm() / base.norm()
+        assert err.item() < 2.0 ** -8
