@@ -693,9 +693,11 @@ extern "C" size_t concord_gemm_workspace_bytes(int64_t M, int64_t N, int64_t K) 
   if (M < 1) M = 1;
   if (N < 1) N = 1;
   if (K < 1) K = 1;
-  const size_t a = splitk_partials(MODE_FWD, M, N, K), b = splitk_partials(MODE_DGRAD, M, K, N),
-               c = splitk_partials(MODE_WGRAD, N, K, M);
-  size_t m = a > b ? (a > c ? a : c) : (b > c ? b : c);
+  // (the first two on a packed or a decoded weight)
+  size_t m = splitk_partials(MODE_WGRAD, N, K, M);
+  for (size_t v : {splitk_partials(MODE_FWD, M, N, K), splitk_partials(MODE_FWD_BF16, M, N, K),
+                   splitk_partials(MODE_DGRAD, M, K, N), splitk_partials(MODE_DGRAD_BF16, M, K, N)})
+    if (v > m) m = v;
   const RaggedRoom r = ragged_room(M, N, K);
   if (r.total) {   // the padded operands, and the partials of the products on them
     const int64_t N8 = ceil8(N), K8 = ceil8(K);

@@ -24,6 +24,7 @@
 //    sums the S fp32 partials in split order.
 #include <algorithm>
 #include <type_traits>
+#include <utility>
 #include <cmath>
 
 #include "gemm.h"
@@ -369,14 +370,6 @@ template <int BI, int BJ, int NT> struct Ops<MODE_FWD, BI, BJ, NT> {
   CONCORD_DEV void init(const GemmArgs& g, int64_t i0, int64_t j0, int t) {
     a.init(g.a + i0 * g.lda, g.lda, g.I - i0, g.R, t);
     b.init(reinterpret_cast<const int32_t*>(g.b) + j0 * g.ldb, g.ldb, g.J - j0, g.R, g.col_exp, t);
-  }
-};
-template <int BI, int BJ, int NT> struct Ops<MODE_FWD_BF16, BI, BJ, NT> {
-  RowsBf16<BI, NT> a;
-  RowsBf16<BJ, NT> b;
-  CONCORD_DEV void init(const GemmArgs& g, int64_t i0, int64_t j0, int t) {
-    a.init(g.a + i0 * g.lda, g.lda, g.I - i0, g.R, t);
-    b.init(reinterpret_cast<const uint16_t*>(g.b) + j0 * g.ldb, g.ldb, g.J - j0, g.R, t);
   }
 };
 template <int BI, int BJ, int NT> struct Ops<MODE_DGRAD, BI, BJ, NT> {
@@ -1761,6 +1754,8 @@ CONCORD_DEV void gemm_tr_body(const GemmArgs& g, const GemmArgs& rd, int tr_bloc
   }
 }
 
+#include "gemm_dd.h"
+
 // LDS bytes of gemm_tr_body's ring
 template <int BI, int BJ>
 constexpr int tr_ring_bytes() { return 3 * (TR * BI * 2 + TR * BJ * 2); }
@@ -2148,6 +2143,56 @@ static FastPlan plan(const FastShape (&shapes)[NS], int64_t I, int64_t J, int64_
   return best;
 }
 
+// The bf16 kernels (gemm_dd_kernel), in us: a block's fixed part (prologue,
+// epilogue, launch) and one TR-deep stage on an otherwise idle chip; both
+// stretch with the share of the CUs at work (clock, L2).  Fitted to the tile
+// shapes and splits of products from 308 x 1280 x 2048 to 4096 x 10240 x 1280
+// run one by one (20 of them, most within 10%): e.g. forward 4096 x 10240 x
+// 1280 took 102.7, 110.2, 122.8 and 105.6 us in 256 x 256, 256 x 128, 192 x 128
+// and 256 x 160 tiles, 2048 x 1280 x 5120 94.9, 48.3, 42.9, 64.6 unsplit and
+// 40.0, 34.8, 34.7, 36.7 at its best split.
+struct DdShape { int bi, bj, waves; double stage; };
+constexpr DdShape kDdShapes[] = {{256, 160, 4, 0.74}, {256, 256, 8, 1.165}, {256, 128, 8, 0.545},
+                                 {192, 128, 4, 0.477}, {128, 128, 4, 0.33}};
+constexpr int kDdCount = 5;
+
+// fwd: the 256 x 160 tile as well (the dgrad's weight tile has 2^n columns).
+// fixed: the split count, 0 to choose it.
+static FastPlan plan_dd(bool fwd, int64_t I, int64_t J, int64_t R, size_t room, bool sym, int fixed) {
+  FastPlan best{kDdCount - 1, 1, 0, 0, R};
+  double best_cost = 1e300;
+  for (int s = fwd ? 0 : 1; s < kDdCount; ++s) {
+    const DdShape& sh = kDdShapes[s];
+    const int64_t ti = cdiv(I, sh.bi), tj = cdiv(J, sh.bj);
+    const int64_t tiles = sym ? sym_tile_count((int)ti, (int)tj, sh.bi, sh.bj) : ti * tj;
+    const double area = (double)sh.bi * sh.bj;
+    const size_t slot = (size_t)(tiles * area) * sizeof(float);
+    const int max_splits = (int)std::min<size_t>(kMaxSplits, std::max<size_t>(1, room / slot));
+    for (int sp = fixed ? fixed : 1; sp <= (fixed ? fixed : max_splits); ++sp) {
+      if (sp > max_splits) break;
+      if (!fixed && sp > 1 && (!gemm_splitk_fits(tiles) || tiles >= kCUs)) break;
+      const int64_t rs = cdiv(cdiv(R, sp), TR) * TR;
+      if (sp > 1 && (sp - 1) * rs >= R) break;
+      const double stages = (double)cdiv(rs, TR);
+      auto round = [&](double fill) {
+        return 4.5 + fill * area / 16384.0 + stages * sh.stage * (1.0 + 0.2 * fill);
+      };
+      const int64_t blocks = tiles * sp, rest = blocks % kCUs;
+      double cost = (double)(blocks / kCUs) * round(1.0) + (rest ? round((double)rest / kCUs) : 0.0);
+      // an unsplit symmetric product's mirrored 2-byte stores (A A, 1280 x 1280
+      // in 128 x 128 tiles: 37 us unsplit, 13 + 5 us split and reduced)
+      if (sym && sp == 1) cost += std::ceil((double)tiles / kCUs) * area * 1.4e-3;
+      // the partials' write and reduction (a symmetric product stores twice)
+      if (sp > 1) cost += 3.0 + (double)sp * (sym ? (double)tiles * area * 2.2e-6 : (double)I * J * 1.4e-6);
+      if (cost < best_cost * 0.999) {
+        best_cost = cost;
+        best = FastPlan{s, sp, (int)ti, (int)tj, rs};
+      }
+    }
+  }
+  return best;
+}
+
 static bool al(const void* p, int n) { return ((uintptr_t)p % n) == 0; }
 // operand extents stay below 2^30 bytes, so kOOB plus any in-tile offset plus
 // the stage's soffset never wraps 32 bits
@@ -2212,6 +2257,12 @@ template <int MODE, int BI, int BJ>
 static void launch_dma(const GemmArgs& g, int blocks, hipStream_t st) {
   hipLaunchKernelGGL((gemm_dma_kernel<MODE, BI, BJ>), dim3(blocks), dim3(512), 0, st, g);
   launch_reduce<MODE, BI, BJ, 2, 2>(g, st);
+}
+
+template <int MODE, int BI, int BJ, int WI, int WJ, int NS>
+static void launch_dd(const GemmArgs& g, int blocks, hipStream_t st) {
+  hipLaunchKernelGGL((gemm_dd_kernel<MODE, BI, BJ, WI, WJ, NS>), dim3(blocks), dim3(64 * WI * WJ), 0, st, g);
+  launch_reduce<MODE, BI, BJ, WI, WJ>(g, st);
 }
 
 template <int BI, int BJ, int WI, int WJ>
@@ -2309,14 +2360,32 @@ static const FastShape& shape_of(int mode, int idx) {
   return kColShapes[idx];
 }
 
+// A layer's product on its decoded weight keeps the splits of the product on
+// the packed weight (the same sums in the same order, so the same bits);
+// symmetric and combined products have no such twin.
+static FastPlan dd_plan(int mode, int64_t I, int64_t J, int64_t R, size_t room, bool sym, bool own) {
+  const bool fwd = mode == MODE_FWD_BF16;
+  const int fixed = own ? 0 : plan_mode(fwd ? MODE_FWD : MODE_DGRAD, I, J, R, room).splits;
+  const FastPlan p = plan_dd(fwd, I, J, R, room, sym, fixed);
+  return p.ti ? p : plan_dd(fwd, I, J, R, room, sym, 0);   // (no room for the fixed splits' partials)
+}
+
 }  // namespace
 
 size_t gemm_fast_partial_bytes(int mode, int64_t I, int64_t J, int64_t R) {
   if (I <= 0 || J <= 0) return 0;
+  size_t bytes = 0;
+  if (mode == MODE_FWD_BF16 || mode == MODE_DGRAD_BF16)
+    for (bool own : {false, true}) {
+      const FastPlan p = dd_plan(mode, I, J, R, (size_t)-1 / 2, false, own);
+      const DdShape& sh = kDdShapes[p.shape];
+      if (p.splits > 1) bytes = std::max(bytes, (size_t)p.ti * p.tj * sh.bi * sh.bj * sizeof(float) * p.splits);
+    }
+  if (mode == MODE_FWD_BF16) return bytes;
   const FastPlan p = plan_mode(mode, I, J, R, (size_t)-1 / 2);
-  if (p.splits <= 1) return 0;
+  if (p.splits <= 1) return bytes;
   const FastShape& sh = shape_of(mode, p.shape);
-  return (size_t)p.ti * p.tj * sh.bi * sh.bj * sizeof(float) * p.splits;
+  return std::max(bytes, (size_t)p.ti * p.tj * sh.bi * sh.bj * sizeof(float) * p.splits);
 }
 
 int64_t gemm_wgrad_vhat_tiles_j(int64_t J) { return cdiv(J, 128); }
@@ -2641,6 +2710,47 @@ int gemm_conv_launch(int mode, const GemmArgs& g0, void* workspace, size_t ws_by
   return launch_status(what);
 }
 
+// FWD_BF16, and DGRAD_BF16 whose weight the DMA's 16-byte chunks can read
+static bool dd_takes(int mode, const GemmArgs& g) {
+  return mode == MODE_FWD_BF16 ||
+         (mode == MODE_DGRAD_BF16 && g.ldb % 8 == 0 && al(g.b, 16) && (g.pad || g.J % 8 == 0));
+}
+
+static int dd_launch(int mode, const GemmArgs& g0, void* workspace, size_t room, hipStream_t st, const char* what,
+                     bool sym) {
+  GemmArgs g = g0;
+  const bool fwd = mode == MODE_FWD_BF16;
+  const FastPlan p = dd_plan(mode, g.I, g.J, g.R, room, sym, sym || g.ay);
+  const DdShape& sh = kDdShapes[p.shape];
+  g.splits = p.splits;
+  g.r_split = p.r_split;
+  g.tiles_i = p.ti;
+  g.tiles_j = p.tj;
+  g.sym = sym ? sym_tile_count(p.ti, p.tj, sh.bi, sh.bj) : 0;
+  if (!sym) g.gi = plan_gi(mode, p, sh.bi, sh.bj);
+  if (p.splits > 1) g.part = (float*)((char*)workspace + kSplitkCounterBytes);
+  const int blocks = (sym ? g.sym : p.ti * p.tj) * p.splits;
+  switch (p.shape) {
+    case 0: launch_dd<MODE_FWD_BF16, 256, 160, 2, 2, 3>(g, blocks, st); break;
+    case 1:
+      if (fwd) launch_dd<MODE_FWD_BF16, 256, 256, 2, 4, 2>(g, blocks, st);
+      else launch_dd<MODE_DGRAD_BF16, 256, 256, 2, 4, 2>(g, blocks, st);
+      break;
+    case 2:
+      if (fwd) launch_dd<MODE_FWD_BF16, 256, 128, 4, 2, 3>(g, blocks, st);
+      else launch_dd<MODE_DGRAD_BF16, 256, 128, 4, 2, 3>(g, blocks, st);
+      break;
+    case 3:
+      if (fwd) launch_dd<MODE_FWD_BF16, 192, 128, 2, 2, 3>(g, blocks, st);
+      else launch_dd<MODE_DGRAD_BF16, 192, 128, 2, 2, 3>(g, blocks, st);
+      break;
+    default:
+      if (fwd) launch_dd<MODE_FWD_BF16, 128, 128, 2, 2, 3>(g, blocks, st);
+      else launch_dd<MODE_DGRAD_BF16, 128, 128, 2, 2, 3>(g, blocks, st);
+  }
+  return launch_status(what);
+}
+
 // sym: the symmetric tile set (FWD / DGRAD modes; the epilogue or the
 // split-K reduction also stores each upper element's mirror image)
 static int fast_launch(int mode, const GemmArgs& g0, void* workspace, size_t ws_bytes, hipStream_t st,
@@ -2649,6 +2759,7 @@ static int fast_launch(int mode, const GemmArgs& g0, void* workspace, size_t ws_
   GemmArgs g = g0;
   // split-K needs room for its partials behind the counters
   const size_t room = (workspace && ws_bytes > kSplitkCounterBytes) ? ws_bytes - kSplitkCounterBytes : 0;
+  if (dd_takes(mode, g)) return dd_launch(mode, g, workspace, room, st, what, sym);
   const FastPlan p = plan_mode(mode, g.I, g.J, g.R, room, sym);
   g.splits = p.splits;
   g.r_split = p.r_split;
@@ -2666,13 +2777,6 @@ static int fast_launch(int mode, const GemmArgs& g0, void* workspace, size_t ws_
       else if (p.shape == 3) launch_dma<MODE_FWD, 192, 160>(g, blocks, st);
       else if (p.shape == 4) launch_dma<MODE_FWD, 192, 128>(g, blocks, st);
       else launch<MODE_FWD, 128, 128, 2, 2, 2>(g, blocks, st);
-      break;
-    case MODE_FWD_BF16:
-      if (p.shape == 0) launch_dma<MODE_FWD_BF16, 256, 160>(g, blocks, st);
-      else if (p.shape == 1) launch_dma<MODE_FWD_BF16, 256, 128>(g, blocks, st);
-      else if (p.shape == 3) launch_dma<MODE_FWD_BF16, 192, 160>(g, blocks, st);
-      else if (p.shape == 4) launch_dma<MODE_FWD_BF16, 192, 128>(g, blocks, st);
-      else launch<MODE_FWD_BF16, 128, 128, 2, 2, 2>(g, blocks, st);
       break;
     case MODE_DGRAD:
       if (p.shape == 0) launch_dgt<MODE_DGRAD, 256, 128>(g, blocks, st);
