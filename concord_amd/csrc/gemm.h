@@ -219,7 +219,8 @@ void vhat_finish_carry_launch(const float* pr, const float* pc, float* bsum, uin
 // tiles along J of the WGRAD launch above (the bias partials' row count)
 int64_t gemm_wgrad_vhat_tiles_j(int64_t J);
 // the other pairing: a split WGRAD with v-hat partials first, then the unsplit
-// dgrad carrying its split-K reduction; -1 when the plans are not of that form
+// dgrad (gd: packed weight, or decoded with row_exp NULL) carrying its split-K
+// reduction; -1 when the plans are not of that form
 int gemm_wgrad_split_dgrad_launch(const GemmArgs& gd, const GemmArgs& gw, void* workspace, size_t ws_bytes,
                                   hipStream_t st, const char* what, int* bias_rows);
 // the products of gemm_dgrad_wgrad_vhat_launch with the v-hat finalize and the
@@ -267,6 +268,8 @@ size_t gemm_conv_partial_bytes(int mode, int64_t I, int64_t J, int64_t R);
 size_t gemm_splitk_need(int mode, int64_t I, int64_t J, int64_t R);
 // split-K partial bytes the fast kernels plan for an I x J x R problem
 // given unlimited workspace (0 when they do not split it)
+// the packed product (MODE_FWD, MODE_DGRAD) runs on a decoded copy of its weight
+bool gemm_decode_pays(int mode, int64_t I, int64_t J, int64_t R);
 size_t gemm_fast_partial_bytes(int mode, int64_t I, int64_t J, int64_t R);
 
 }  // namespace concord

@@ -582,6 +582,32 @@ static void ragged_wgrad(const Ragged& rg, GemmArgs& g) {
   g.sc = ragged_out(g);
 }
 
+// room of a layer's decoded weight (0: neither product decodes)
+static size_t decode_room(int64_t M, int64_t N, int64_t K) {
+  if (!gemm_decode_pays(MODE_FWD, M, N, K) && !gemm_decode_pays(MODE_DGRAD, M, K, N)) return 0;
+  return round256((size_t)N * (size_t)K * 2);
+}
+
+// g (forward or dgrad on packed words) as the product on the decoded weight,
+// decoded into the end of the workspace (`inner` bytes stay before it); false
+// where decoding does not pay, does not fit, or the bf16 kernel would not take it
+static bool decoded(int mode, const GemmArgs& g, void* workspace, size_t ws_bytes, hipStream_t st, GemmArgs& out,
+                    size_t& inner, int& rc) {
+  if (!gemm_decode_pays(mode, g.I, g.J, g.R) || !workspace || !gemm_fast_takes(mode, g)) return false;
+  const int64_t N = mode == MODE_FWD ? g.J : g.R, K = mode == MODE_FWD ? g.R : g.J;
+  const size_t room = round256((size_t)N * (size_t)K * 2);
+  if (ws_bytes < kSplitkCounterBytes + room + 256) return false;
+  inner = (ws_bytes - room) / 256 * 256;
+  uint16_t* w = (uint16_t*)((char*)workspace + inner);
+  out = g;
+  out.b = w;
+  out.ldb = K;
+  out.row_exp = out.col_exp = nullptr;
+  if (!gemm_fast_takes(mode == MODE_FWD ? MODE_FWD_BF16 : MODE_DGRAD_BF16, out)) return false;
+  rc = concord_materialize((const int32_t*)g.b, g.ldb, g.row_exp, g.col_exp, N, K, g.bias, 0, w, K, st);
+  return true;
+}
+
 template <int MODE>
 static int launch_gemm(GemmArgs g, void* workspace, size_t ws_bytes, hipStream_t st,
                        const char* what) {
@@ -601,9 +627,23 @@ static int launch_gemm(GemmArgs g, void* workspace, size_t ws_bytes, hipStream_t
       if (rc != -1) return rc;
     }
   }
+  if constexpr (MODE == MODE_FWD || MODE == MODE_DGRAD) {
+    GemmArgs d;
+    size_t inner = 0;
+    int rc = CONCORD_OK;
+    if (decoded(MODE, g, workspace, ws_bytes, st, d, inner, rc))
+      return rc != CONCORD_OK ? rc
+                              : gemm_fast_launch(MODE == MODE_FWD ? MODE_FWD_BF16 : MODE_DGRAD_BF16, d, workspace,
+                                                 inner, st, what);
+  }
   const int fast = gemm_fast_launch(MODE, g, workspace, ws_bytes, st, what);
   if (fast != -1) return fast;
-  const bool can_split = workspace != nullptr;
+  // the tile counters of a split launch start at zero; a layer with a decoded
+  // weight may pass a fresh workspace
+  const bool can_split = workspace != nullptr &&
+                         (MODE == MODE_WGRAD            ? decode_room(g.R, g.I, g.J)
+                          : MODE == MODE_FWD || MODE == MODE_FWD_BF16 ? decode_room(g.I, g.J, g.R)
+                                                        : decode_room(g.I, g.R, g.J)) == 0;
   Plan p = plan_gemm(g.I, g.J, g.R, can_split);
   if (p.splits == 2 &&
       (ws_bytes < gemm_splitk_bytes(g.I, g.J) || !gemm_splitk_fits((int64_t)p.ti * p.tj)))
@@ -705,7 +745,12 @@ extern "C" size_t concord_gemm_workspace_bytes(int64_t M, int64_t N, int64_t K) 
       if (v > m) m = v;
     m = round256(m) + r.total + 256;
   }
+  if (const size_t w = decode_room(M, N, K)) m = round256(m) + w + 256;
   return kSplitkCounterBytes + ((m + 255) / 256) * 256;
+}
+
+extern "C" int concord_gemm_decodes_weight(int64_t M, int64_t N, int64_t K) {
+  return M > 0 && N > 0 && K > 0 && decode_room(M, N, K) != 0;
 }
 
 extern "C" int concord_dqgemm_fwd(const uint16_t* x, int64_t ld_x, const int32_t* packed,
@@ -800,7 +845,20 @@ static int wgrad_vhat_impl(const GemmArgs* gd, const uint16_t* dy, int64_t ld_dy
     gemm_workspace_bytes = rg.inner;
     gd = nullptr;
   }
-  if (gd && gd->I > 0 && gd->J > 0) {
+  GemmArgs dec;
+  size_t dec_inner = 0;
+  int dec_rc = CONCORD_OK;
+  if (gd && gd->I > 0 && gd->J > 0 &&
+      decoded(MODE_DGRAD, *gd, gemm_workspace, gemm_workspace_bytes, st, dec, dec_inner, dec_rc)) {
+    if (dec_rc != CONCORD_OK) return dec_rc;
+    gemm_workspace_bytes = dec_inner;
+    rc = gemm_wgrad_split_dgrad_launch(dec, g, gemm_workspace, dec_inner, st, what, &tiles_j);
+    if (rc == -1) {
+      rc = gemm_fast_launch(MODE_DGRAD_BF16, dec, gemm_workspace, dec_inner, st, what);
+      if (rc != CONCORD_OK) return rc;
+      rc = -1;
+    }
+  } else if (gd && gd->I > 0 && gd->J > 0) {
     rc = gemm_dgrad_wgrad_vhat_launch(*gd, gemm_workspace, gemm_workspace ? gemm_workspace_bytes : 0, g, st,
                                       what, &tiles_j, &pend, &pend_rbi);
     if (rc == -1)

@@ -256,14 +256,25 @@ CONCORD_DEV void dd_loop(f32x4 (&acc)[NI][NJ], const SA& sa, const SB& sb, int64
 // 8192 x 640 x 5120 67.5 -> 51.3, 4096 x 1280 x 1280 21.8 -> 18.0; forward
 // 4096 x 10240 x 1280 113.6 -> 109.1, 4096 x 1280 x 1280 22.0 -> 18.5,
 // 2048 x 1280 x 5120 40.4 -> 35.0.
-template <int MODE, int BI, int BJ, int WI, int WJ, int NS>
-__global__ __launch_bounds__(64 * WI * WJ, 1) void gemm_dd_kernel(GemmArgs g) {
+//
+// CARRY (8 waves): workgroups from dg_blocks on run the v-hat reduction of the
+// split WGRAD rw issued just before on the stream, on the CUs the tiles leave
+// idle, two reduction blocks at a time.
+template <int MODE, int BI, int BJ, int WI, int WJ, int NS, bool CARRY = false>
+__global__ __launch_bounds__(64 * WI * WJ, 1) void gemm_dd_kernel(GemmArgs g, GemmArgs rw, int dg_blocks) {
   constexpr int NW = WI * WJ, WTI = BI / WI, WTJ = BJ / WJ, NI = WTI / 16, NJ = WTJ / 16;
   constexpr bool FWD = MODE == MODE_FWD_BF16;
   typedef DdRows<BI, WTI, NW> SA;
   typedef typename std::conditional<FWD, DdRows<BJ, WTJ, NW>, DdCols<BJ, WTJ, NW>>::type SB;
   constexpr int RING = NS * (SA::TILE + SB::TILE), OUT = BI * (BJ + 8) * 2;
   __shared__ __attribute__((aligned(1024))) char lds[RING > OUT ? RING : OUT];
+  if constexpr (CARRY) {
+    if ((int)blockIdx.x >= dg_blocks) {
+      ReduceVh<256, 128, 4, 2>::run_pairs(rw, (int)blockIdx.x - dg_blocks, (int)gridDim.x - dg_blocks,
+                                          reinterpret_cast<float*>(lds));
+      return;
+    }
+  }
   const int t = threadIdx.x, lane = t & 63, wave = __builtin_amdgcn_readfirstlane(t >> 6);
   int split, bi, bj, slot;
   gemm_tile_of<BI, BJ>(g, blockIdx.x, split, bi, bj, slot);

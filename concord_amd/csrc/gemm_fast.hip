@@ -804,6 +804,20 @@ struct ReduceVh {
         for (int e = 0; e < 4; ++e) g2[xx][y][e] = s_g2[((xx * NJ + y) * 4 + e) * 64 + lane];
     vhat_tile_partials(g2, lane, row0, col0, g.I, g.J, g.vh_pr, g.vh_pc);
   }
+  // all blocks of the reduction on `ngroups` workgroups of 512 threads, two
+  // blocks at a time; s_g2: 2 x LDS_FLOATS
+  static CONCORD_DEV void run_pairs(const GemmArgs& g, int group, int ngroups, float* s_g2) {
+    const int nblk = g.tiles_i * g.tiles_j * NAW;
+    const int half = threadIdx.x >> 8, tid = threadIdx.x & 255;
+    s_g2 += half * LDS_FLOATS;
+    for (int b0 = 2 * group; b0 < nblk; b0 += 2 * ngroups) {
+      const int blk = b0 + half;
+      if (blk < nblk) part1(g, blk, tid, s_g2);
+      __syncthreads();
+      if (blk < nblk) part2(g, blk, tid, s_g2);
+      __syncthreads();   // s_g2 is reused by the next pair
+    }
+  }
 };
 
 template <int BI, int BJ, int WI, int WJ>
@@ -1919,17 +1933,7 @@ CONCORD_DEV void gemm_dgt_body(const GemmArgs& g, const GemmArgs& rw, int dg_blo
     typedef ReduceVh<256, 128, 4, 2> RV;
     static_assert(sizeof(lds_a) >= 2 * RV::LDS_FLOATS * sizeof(float), "two reduction blocks fit");
     if (wg >= dg_blocks) {
-      const int nblk = rw.tiles_i * rw.tiles_j * RV::NAW;
-      const int half = threadIdx.x >> 8, tid = threadIdx.x & 255;
-      float* s_g2 = reinterpret_cast<float*>(&lds_a[0][0]) + half * RV::LDS_FLOATS;
-      const int stride = 2 * (ngrid - dg_blocks);
-      for (int b0 = 2 * (wg - dg_blocks); b0 < nblk; b0 += stride) {
-        const int blk = b0 + half;
-        if (blk < nblk) RV::part1(rw, blk, tid, s_g2);
-        __syncthreads();
-        if (blk < nblk) RV::part2(rw, blk, tid, s_g2);
-        __syncthreads();   // s_g2 is reused by the next pair
-      }
+      RV::run_pairs(rw, wg - dg_blocks, ngrid - dg_blocks, reinterpret_cast<float*>(&lds_a[0][0]));
       return;
     }
   }
@@ -2151,9 +2155,9 @@ static FastPlan plan(const FastShape (&shapes)[NS], int64_t I, int64_t J, int64_
 // 1280 took 102.7, 110.2, 122.8 and 105.6 us in 256 x 256, 256 x 128, 192 x 128
 // and 256 x 160 tiles, 2048 x 1280 x 5120 94.9, 48.3, 42.9, 64.6 unsplit and
 // 40.0, 34.8, 34.7, 36.7 at its best split.
-struct DdShape { int bi, bj, waves; double stage; };
-constexpr DdShape kDdShapes[] = {{256, 160, 4, 0.74}, {256, 256, 8, 1.165}, {256, 128, 8, 0.545},
-                                 {192, 128, 4, 0.477}, {128, 128, 4, 0.33}};
+struct DdShape { int bi, bj, waves; double stage, full; };   // full: the fixed part's growth on a full chip
+constexpr DdShape kDdShapes[] = {{256, 160, 4, 0.74, 4.0}, {256, 256, 8, 1.165, 4.0}, {256, 128, 8, 0.545, 4.0},
+                                 {192, 128, 4, 0.477, 2.0}, {128, 128, 4, 0.33, 1.5}};
 constexpr int kDdCount = 5;
 
 // fwd: the 256 x 160 tile as well (the dgrad's weight tile has 2^n columns).
@@ -2175,7 +2179,7 @@ static FastPlan plan_dd(bool fwd, int64_t I, int64_t J, int64_t R, size_t room, 
       if (sp > 1 && (sp - 1) * rs >= R) break;
       const double stages = (double)cdiv(rs, TR);
       auto round = [&](double fill) {
-        return 4.5 + fill * area / 16384.0 + stages * sh.stage * (1.0 + 0.2 * fill);
+        return 4.5 + fill * sh.full + stages * sh.stage * (1.0 + 0.2 * fill);
       };
       const int64_t blocks = tiles * sp, rest = blocks % kCUs;
       double cost = (double)(blocks / kCUs) * round(1.0) + (rest ? round((double)rest / kCUs) : 0.0);
@@ -2261,7 +2265,8 @@ static void launch_dma(const GemmArgs& g, int blocks, hipStream_t st) {
 
 template <int MODE, int BI, int BJ, int WI, int WJ, int NS>
 static void launch_dd(const GemmArgs& g, int blocks, hipStream_t st) {
-  hipLaunchKernelGGL((gemm_dd_kernel<MODE, BI, BJ, WI, WJ, NS>), dim3(blocks), dim3(64 * WI * WJ), 0, st, g);
+  hipLaunchKernelGGL((gemm_dd_kernel<MODE, BI, BJ, WI, WJ, NS>), dim3(blocks), dim3(64 * WI * WJ), 0, st, g,
+                     GemmArgs{}, blocks);
   launch_reduce<MODE, BI, BJ, WI, WJ>(g, st);
 }
 
@@ -2360,6 +2365,12 @@ static const FastShape& shape_of(int mode, int idx) {
   return kColShapes[idx];
 }
 
+// FWD_BF16, and DGRAD_BF16 whose weight the DMA's 16-byte chunks can read
+static bool dd_takes(int mode, const GemmArgs& g) {
+  return mode == MODE_FWD_BF16 ||
+         (mode == MODE_DGRAD_BF16 && g.ldb % 8 == 0 && al(g.b, 16) && (g.pad || g.J % 8 == 0));
+}
+
 // A layer's product on its decoded weight keeps the splits of the product on
 // the packed weight (the same sums in the same order, so the same bits);
 // symmetric and combined products have no such twin.
@@ -2386,6 +2397,25 @@ size_t gemm_fast_partial_bytes(int mode, int64_t I, int64_t J, int64_t R) {
   if (p.splits <= 1) return bytes;
   const FastShape& sh = shape_of(mode, p.shape);
   return std::max(bytes, (size_t)p.ti * p.tj * sh.bi * sh.bj * sizeof(float) * p.splits);
+}
+
+// Decode first (one pass over the weight, ~2.2 us + 0.85 us per 2^20 words) and
+// run the bf16 kernel, instead of decoding in the product's producer waves,
+// which bound its stages: worth it once enough row tiles share the weight.
+// dgrad, packed kernel -> decode + bf16 kernel, us: 4096 x 1280 x 10240 138 ->
+// 109, 16384 x 640 x 640 29.5 -> 23.8, 8192 x 640 x 5120 71.7 -> 56.8,
+// 2048 x 5120 x 1280 45.2 -> 39.0 (training steps of those layers 2 - 6%
+// shorter).  Forward: 8192 x 5120 x 640 82.6 -> 67.6, but training steps whose
+// forward also decoded were 1 - 3% longer at 4096 x 1280 x 1280,
+// 4096 x 10240 x 1280 and 16384 x 640 x 640, where the pass reads a weight no
+// cache holds and the chip's clock, not the producers, sets the product's pace.
+// Below 4e9 products the pass's fixed time takes the gain.  A split dgrad
+// keeps the packed kernel: the WGRAD launch carries its reduction
+// (2048 x 1280 x 5120: 42.8 -> 42 without that).
+bool gemm_decode_pays(int mode, int64_t I, int64_t J, int64_t R) {
+  if ((double)I * (double)J * (double)R < 4e9 || J % 8 != 0 || R % 8 != 0) return false;
+  if (mode == MODE_FWD) return I >= 8192 && (double)I * (double)J * (double)R >= 1.6e10;
+  return mode == MODE_DGRAD && I >= 2048 && plan_mode(mode, I, J, R, (size_t)-1 / 2).splits == 1;
 }
 
 int64_t gemm_wgrad_vhat_tiles_j(int64_t J) { return cdiv(J, 128); }
@@ -2469,12 +2499,16 @@ static FastPlan carry_dgrad_shape(const FastPlan& pd, int64_t I, int64_t R, int 
 
 int gemm_wgrad_split_dgrad_launch(const GemmArgs& gd0, const GemmArgs& gw0, void* workspace, size_t ws_bytes,
                                   hipStream_t st, const char* what, int* bias_rows) {
-  if (!eligible(MODE_DGRAD, gd0) || !eligible(MODE_WGRAD, gw0) || !tr_eligible(gw0) || !workspace) return -1;
+  // a decoded weight (no exponents): the bf16 kernel's tiles
+  const bool dec = gd0.row_exp == nullptr;
+  if (!eligible(dec ? MODE_DGRAD_BF16 : MODE_DGRAD, gd0) || (dec && !dd_takes(MODE_DGRAD_BF16, gd0)) || !eligible(MODE_WGRAD, gw0) || !tr_eligible(gw0) || !workspace) return -1;
   const size_t room = ws_bytes > kSplitkCounterBytes ? ws_bytes - kSplitkCounterBytes : 0;
   FastPlan pd = plan_mode(MODE_DGRAD, gd0.I, gd0.J, gd0.R, room);
   const FastPlan pw = plan_mode(MODE_WGRAD, gw0.I, gw0.J, gw0.R, room);
   if ((pd.shape != 0 && pd.shape != 2) || pd.splits != 1 || pw.shape != 0 || pw.splits < 2) return -1;
-  pd = carry_dgrad_shape(pd, gd0.I, gd0.R, pw.ti * pw.tj * 8);
+  // (decoded: the 8-wave 256 x 128 tile, whose workgroups the reduction's size fits)
+  if (dec) pd = FastPlan{0, 1, (int)cdiv(gd0.I, 256), (int)cdiv(gd0.J, 128), pd.r_split};
+  else pd = carry_dgrad_shape(pd, gd0.I, gd0.R, pw.ti * pw.tj * 8);
   const int td = pd.ti * pd.tj;
   const int extra = kCUs - td;
   if (extra < 16) return -1;   // the dgrad grid leaves too few CUs to carry the reduction
@@ -2490,12 +2524,15 @@ int gemm_wgrad_split_dgrad_launch(const GemmArgs& gd0, const GemmArgs& gw0, void
   gd.r_split = pd.r_split;
   gd.tiles_i = pd.ti;
   gd.tiles_j = pd.tj;
-  gd.gi = plan_gi(MODE_DGRAD, pd, pd.shape == 0 ? 256 : 192, 128);
+  gd.gi = plan_gi(dec ? MODE_DGRAD_BF16 : MODE_DGRAD, pd, pd.shape == 0 ? 256 : 192, 128);
   *bias_rows = pw.tj;
   const int tiles = pw.ti * pw.tj;
   hipLaunchKernelGGL((gemm_tr_kernel<256, 128, 4, 2, false>), dim3(tiles * pw.splits), dim3(512), 0, st, gw,
                      GemmArgs{}, tiles * pw.splits);
-  if (pd.shape == 0)
+  if (dec)
+    hipLaunchKernelGGL((gemm_dd_kernel<MODE_DGRAD_BF16, 256, 128, 4, 2, 3, true>), dim3(td + extra), dim3(512), 0, st,
+                       gd, gw, td);
+  else if (pd.shape == 0)
     hipLaunchKernelGGL((gemm_dgt_carry_kernel<256, 128>), dim3(td + extra), dim3(512), 0, st, gd, gw, td);
   else
     hipLaunchKernelGGL((gemm_dgt_carry_kernel<192, 128>), dim3(td + extra), dim3(512), 0, st, gd, gw, td);
@@ -2708,12 +2745,6 @@ int gemm_conv_launch(int mode, const GemmArgs& g0, void* workspace, size_t ws_by
       return -1;
   }
   return launch_status(what);
-}
-
-// FWD_BF16, and DGRAD_BF16 whose weight the DMA's 16-byte chunks can read
-static bool dd_takes(int mode, const GemmArgs& g) {
-  return mode == MODE_FWD_BF16 ||
-         (mode == MODE_DGRAD_BF16 && g.ldb % 8 == 0 && al(g.b, 16) && (g.pad || g.J % 8 == 0));
 }
 
 static int dd_launch(int mode, const GemmArgs& g0, void* workspace, size_t room, hipStream_t st, const char* what,

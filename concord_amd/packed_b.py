@@ -229,9 +229,13 @@ _GEMM_WORKSPACES = {}
 
 def _gemm_workspace(device, M, N, K):
     """Zero-initialised per-device split-K workspace of the GEMMs, grown to the
-    largest problem seen (grow it eagerly, before any graph capture)."""
+    largest problem seen (grow it eagerly, before any graph capture).  A layer
+    whose products decode the weight into the workspace gets its own from the
+    allocator: forwards on several streams must not share it."""
     key = _dev_key(device)
     need = int(C.lib().concord_gemm_workspace_bytes(int(M), int(N), int(K)))
+    if C.lib().concord_gemm_decodes_weight(int(M), int(N), int(K)):
+        return torch.empty(need, dtype=torch.uint8, device=key)
     ws = _GEMM_WORKSPACES.get(key)
     if ws is None or ws.numel() < need:
         ws = torch.zeros(need, dtype=torch.uint8, device=key)

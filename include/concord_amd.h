@@ -211,6 +211,10 @@ int concord_load_weights(const float* W, int64_t ld_w, int64_t N, int64_t K, int
  * 2-way along the reduction and the halves are added in a fixed way
  * (bit-identical whichever half finishes first). */
 size_t concord_gemm_workspace_bytes(int64_t M, int64_t N, int64_t K);
+/* 1 where the layer's large products decode the packed weight once into the
+ * workspace (its last bytes) instead of in every tile.  Such a layer's calls
+ * need no zero-filled workspace, and may each take a fresh one. */
+int concord_gemm_decodes_weight(int64_t M, int64_t N, int64_t K);
 
 /* Dequant-GEMM forward: y[M,N] = x[M,K] . decode(packed)[N,K]^T (+ bias[N]),
  * bf16 in/out, fp32 accumulation on bf16 MFMA.  Replaces

@@ -36,3 +36,30 @@ def test_bf16_products(M, N, K):
         # one rounding to bf16 (2^-8 of the value) and R fp32 additions
         bound = ref.abs() * 2.0 ** -8 + mag * R * 2.0 ** -24
         assert torch.all((got.double() - ref).abs() <= bound)
+
+
+@pytest.mark.parametrize("M,N,K", [(4096, 1280, 1280), (4104, 1288, 1272), (2048, 1280, 5120), (4096, 640, 2560),
+                                   (2056, 5128, 1288), (16384, 640, 640), (8200, 2568, 1272)])
+def test_packed_products_on_a_decoded_copy(M, N, K):
+    """Large packed products decode the weight first: the bits of the product
+    on the materialised weight (power-of-two scales, same sums), in the
+    separate and the combined backward entry."""
+    import concord_amd as ca
+    from concord_amd import packed_b as pb
+    torch.manual_seed(N)
+    la = ca.ConcordLinearPackedB(K, N, bias=True, device="cuda", lr=5e-4)
+    x = torch.randn(M, K, device="cuda").bfloat16()
+    dy = (torch.randn(M, N, device="cuda") * 1e-3).bfloat16()
+    W = la.get_weight()
+    la.bias.data.normal_()
+    args = (la.packed_w, la.row_exp, la.col_exp, 15)
+    y = pb._gemm_fwd(x, *args, la.bias, None)
+    assert torch.equal(y, pb._gemm_fwd(x, None, None, None, 15, la.bias, W))
+    dx = pb._gemm_dgrad(dy, *args, None)
+    assert torch.equal(dx, pb._gemm_dgrad(dy, None, None, None, 15, W))
+    gw = pb._wgrad(dy, x)
+    dx2, gw2, gb2 = pb._dgrad_wgrad_vhat(dy, x, *args, la.v_row, la.v_col, la._sum_v_inv, 0.999, la._row_max_buf,
+                                         la._col_max_buf, pb._get_step_counter("cuda"), True)
+    assert torch.equal(dx, dx2) and torch.equal(gw, gw2)
+    ref = dy.double().sum(0)
+    assert torch.all((gb2.double() - ref).abs() <= ref.abs() * 2.0 ** -8 + dy.double().abs().sum(0) * M * 2.0 ** -24)
