@@ -458,9 +458,15 @@ CONCORD_DEV float* partial_slot(const GemmArgs& g, int tile, int split, int aw) 
   return g.part + ((int64_t)tile * g.splits + split) * ((int64_t)NAW * NI * NJ * 256) + (int64_t)aw * NI * NJ * 256;
 }
 
+// products that may have a ragged output (g.sc): the packed modes do not
+// (their split-K reduction measured 0.4 us longer with the branch)
+template <int MODE>
+constexpr bool ragged_mode() { return MODE != MODE_FWD && MODE != MODE_DGRAD; }
+
 // the bias of columns j .. j + 3 (j < J)
+template <int MODE>
 CONCORD_DEV void load_bias4(const GemmArgs& g, int64_t j, float (&bs)[4]) {
-  if (g.sc) {
+  if (ragged_mode<MODE>() && g.sc) {
 #pragma unroll
     for (int e = 0; e < 4; ++e) bs[e] = j + e < g.J ? bf16_to_f32(g.vbias[j + e]) : 0.f;
     return;
@@ -473,9 +479,10 @@ CONCORD_DEV void load_bias4(const GemmArgs& g, int64_t j, float (&bs)[4]) {
 }
 
 // 4 bf16 (o) to columns j .. j + 3 of an output row (j < J)
+template <int MODE>
 CONCORD_DEV void store4(const GemmArgs& g, int64_t i, int64_t j, uint2 o) {
   uint16_t* c = g.c + i * g.ldc + j;
-  if (!g.sc) {
+  if (!ragged_mode<MODE>() || !g.sc) {
     *reinterpret_cast<uint2*>(c) = o;
     return;
   }
@@ -516,7 +523,7 @@ CONCORD_DEV void epilogue(const GemmArgs& g, f32x4 (&acc)[NI][NJ], int64_t i0, i
 #pragma unroll
           for (int e = 0; e < 4; ++e) sc[e] = exp2i(sbyte(e4, e) - g.bias);
         }
-        if (g.vbias) load_bias4(g, j, bs);
+        if (g.vbias) load_bias4<MODE>(g, j, bs);
       }
 #pragma unroll
       for (int x = 0; x < NI; ++x) {
@@ -533,7 +540,7 @@ CONCORD_DEV void epilogue(const GemmArgs& g, f32x4 (&acc)[NI][NJ], int64_t i0, i
   // row-contiguous stores: 8 bf16 (16 bytes) per thread when the output
   // allows, else 4 (J % 4 == 0, ldc % 4 == 0, 8-byte aligned base)
   const bool v16 = (g.ldc % 8 == 0) && (g.J % 8 == 0) && (((uintptr_t)g.c % 16) == 0);
-  if (g.sc) {
+  if (ragged_mode<MODE>() && g.sc) {
     // ragged rows: one element per thread, consecutive threads consecutive columns
     for (int c = t; c < BI * BJ; c += nthreads) {
       const int rl = c / BJ, cl = c % BJ;
@@ -627,7 +634,7 @@ CONCORD_DEV void splitk_reduce_item_sp(const GemmArgs& g, int64_t idx) {
 #pragma unroll
     for (int e = 0; e < 4; ++e) sc[e] = exp2i(sbyte(e4, e) - g.bias);
   }
-  if (g.vbias) load_bias4(g, j, bs);
+  if (g.vbias) load_bias4<MODE>(g, j, bs);
   float v[4];
 #pragma unroll
   for (int e = 0; e < 4; ++e) v[e] = __fadd_rn(__fmul_rn(sum[e], sc[e]), bs[e]);
@@ -652,7 +659,7 @@ CONCORD_DEV void splitk_reduce_item_sp(const GemmArgs& g, int64_t idx) {
     }
     return;
   }
-  store4(g, i, j, o);
+  store4<MODE>(g, i, j, o);
 }
 
 // splitk_reduce_item_sp for the launch's split count (uniform), 2 .. kGemmMaxSplits
@@ -766,7 +773,7 @@ struct ReduceVh {
 #pragma unroll
         for (int e = 0; e < 4; ++e) s_g2[((x * NJ + y) * 4 + e) * 64 + lane] = __fmul_rn(v[e], v[e]);
         const int64_t i = row0 + x * 16 + (lane & 15), j = col0 + y * 16 + 4 * (lane >> 4);
-        if (i < g.I && j < g.J) store4(g, i, j, make_uint2(lo, hi));
+        if (i < g.I && j < g.J) store4<MODE_WGRAD>(g, i, j, make_uint2(lo, hi));
       }
     }
     if (x == 1 && g.bpart && aw % WJ == 0) {
