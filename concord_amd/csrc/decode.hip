@@ -9,9 +9,33 @@
 
 namespace concord {
 
-// A lane decodes 8 consecutive words (two 16 B loads, one 16 B store); a
-// block of 256 lanes covers 2048 columns of rows blockIdx.y, blockIdx.y +
-// gridDim.y, ...
+// 8 consecutive words (two 16 B loads, one 16 B store; k0 + 8 <= K columns or
+// fewer) of one row
+template <bool CONSOLIDATED, bool VEC>
+CONCORD_DEV void decode8(const int32_t* __restrict__ src, uint16_t* __restrict__ dst, int32_t te_row,
+                         const int8_t* col_exp, int64_t k0, int64_t K) {
+  auto decode = [&](int32_t w, int64_t k) -> float {
+    const Fields f = unpack(w);
+    const int32_t m = CONSOLIDATED ? (f.ss + f.vs) * 128 : f.ss * 128 + f.sf + f.vs * 128;
+    return __fmul_rn((float)m, exp2i(te_row + (int32_t)col_exp[k]));
+  };
+  if (VEC && k0 + 8 <= K) {
+    const int4 a = *reinterpret_cast<const int4*>(src);
+    const int4 b = *reinterpret_cast<const int4*>(src + 4);
+    uint4 o;
+    o.x = pack_bf16x2(decode(a.x, k0 + 0), decode(a.y, k0 + 1));
+    o.y = pack_bf16x2(decode(a.z, k0 + 2), decode(a.w, k0 + 3));
+    o.z = pack_bf16x2(decode(b.x, k0 + 4), decode(b.y, k0 + 5));
+    o.w = pack_bf16x2(decode(b.z, k0 + 6), decode(b.w, k0 + 7));
+    *reinterpret_cast<uint4*>(dst) = o;
+  } else {
+    for (int j = 0; j < 8 && k0 + j < K; ++j)
+      dst[j] = (uint16_t)(pack_bf16x2(decode(src[j], k0 + j), 0.0f) & 0xFFFFu);
+  }
+}
+
+// A lane decodes 8 words; a block of 256 lanes covers 2048 columns of rows
+// blockIdx.y, blockIdx.y + gridDim.y, ...
 template <bool CONSOLIDATED, bool VEC>
 __global__ __launch_bounds__(256) void materialize_kernel(const int32_t* __restrict__ packed,
                                                           int64_t ld_p, const int8_t* row_exp,
@@ -21,28 +45,60 @@ __global__ __launch_bounds__(256) void materialize_kernel(const int32_t* __restr
                                                           int64_t ld_o) {
   const int64_t k0 = ((int64_t)blockIdx.x * 256 + threadIdx.x) * 8;
   if (k0 >= K) return;
-  for (int64_t n = blockIdx.y; n < N; n += gridDim.y) {
-    const int32_t te_row = (int32_t)row_exp[n] - bias;
-    const int32_t* src = packed + n * ld_p + k0;
-    uint16_t* dst = out + n * ld_o + k0;
-    auto decode = [&](int32_t w, int64_t k) -> float {
-      const Fields f = unpack(w);
-      const int32_t m = CONSOLIDATED ? (f.ss + f.vs) * 128 : f.ss * 128 + f.sf + f.vs * 128;
-      return __fmul_rn((float)m, exp2i(te_row + (int32_t)col_exp[k]));
-    };
-    if (VEC && k0 + 8 <= K) {
-      const int4 a = *reinterpret_cast<const int4*>(src);
-      const int4 b = *reinterpret_cast<const int4*>(src + 4);
-      uint4 o;
-      o.x = pack_bf16x2(decode(a.x, k0 + 0), decode(a.y, k0 + 1));
-      o.y = pack_bf16x2(decode(a.z, k0 + 2), decode(a.w, k0 + 3));
-      o.z = pack_bf16x2(decode(b.x, k0 + 4), decode(b.y, k0 + 5));
-      o.w = pack_bf16x2(decode(b.z, k0 + 6), decode(b.w, k0 + 7));
-      *reinterpret_cast<uint4*>(dst) = o;
-    } else {
-      for (int j = 0; j < 8 && k0 + j < K; ++j)
-        dst[j] = (uint16_t)(pack_bf16x2(decode(src[j], k0 + j), 0.0f) & 0xFFFFu);
+  for (int64_t n = blockIdx.y; n < N; n += gridDim.y)
+    decode8<CONSOLIDATED, VEC>(packed + n * ld_p + k0, out + n * ld_o + k0, (int32_t)row_exp[n] - bias, col_exp, k0, K);
+}
+
+// Many layers in one launch (an export is launch bound: 5.3 us of kernel in
+// ~20 us of host time a layer).  A block takes 1024 chunks of 8 words of one
+// item, counted through its rows, so no lane idles on a short row; it finds
+// its item by the items' first blocks.
+constexpr int kGroupItems = 24, kGroupChunks = 1024;
+struct GroupItem {
+  const int32_t* packed;   // nullptr: copy `chunks` pieces of 8 bytes and `tail` bytes
+  const int8_t* row_exp;
+  const int8_t* col_exp;
+  uint16_t* out;
+  int64_t ld_p, ld_o, K;
+  uint32_t chunks, cpr, first;   // cpr: chunks per row
+  int32_t bias;
+  int32_t vec, tail;
+};
+struct Group {
+  GroupItem it[kGroupItems];
+  int n;
+};
+
+template <bool CONSOLIDATED>
+__global__ __launch_bounds__(256) void materialize_group_kernel(Group g) {
+  int i = 0;
+  while (i + 1 < g.n && blockIdx.x >= g.it[i + 1].first) ++i;
+  const GroupItem& t = g.it[i];
+  const uint32_t q0 = (blockIdx.x - t.first) * kGroupChunks + threadIdx.x;
+  if (!t.packed) {
+    const uint8_t* src = reinterpret_cast<const uint8_t*>(t.row_exp);
+    uint8_t* dst = reinterpret_cast<uint8_t*>(t.out);
+#pragma unroll
+    for (int u = 0; u < kGroupChunks / 256; ++u) {
+      const uint32_t q = q0 + u * 256;
+      if (q >= t.chunks) break;
+      const int left = q + 1 == t.chunks ? t.tail : 8;
+      if (t.vec && left == 8) *reinterpret_cast<uint2*>(dst + (int64_t)q * 8) = *reinterpret_cast<const uint2*>(src + (int64_t)q * 8);
+      else for (int e = 0; e < left; ++e) dst[(int64_t)q * 8 + e] = src[(int64_t)q * 8 + e];
     }
+    return;
+  }
+#pragma unroll
+  for (int u = 0; u < kGroupChunks / 256; ++u) {
+    const uint32_t q = q0 + u * 256;
+    if (q >= t.chunks) break;
+    const uint32_t n = q / t.cpr;
+    const int64_t k0 = (int64_t)(q - n * t.cpr) * 8;
+    const int32_t* src = t.packed + (int64_t)n * t.ld_p + k0;
+    uint16_t* dst = t.out + (int64_t)n * t.ld_o + k0;
+    const int32_t te = (int32_t)t.row_exp[n] - t.bias;
+    if (t.vec) decode8<CONSOLIDATED, true>(src, dst, te, t.col_exp, k0, t.K);
+    else decode8<CONSOLIDATED, false>(src, dst, te, t.col_exp, k0, t.K);
   }
 }
 
@@ -139,6 +195,61 @@ extern "C" int concord_materialize(const int32_t* packed, int64_t ld_p, const in
   }
 #undef LAUNCH
   return launch_status("materialize");
+}
+
+extern "C" int concord_materialize_group(const concord_materialize_item* items, int32_t n, int consolidated,
+                                         void* stream) {
+  CONCORD_CHECK(n >= 0 && (items || n == 0), "concord_materialize_group: bad argument");
+  for (int32_t i = 0; i < n; ++i) {
+    const concord_materialize_item& a = items[i];
+    CONCORD_CHECK(a.N >= 0 && a.K >= 0 && a.N <= (1LL << 31) && a.K < (1LL << 31),
+                  "concord_materialize_group: bad size");
+    if (a.N == 0 || a.K == 0) continue;
+    CONCORD_CHECK(a.row_exp && a.out && (!a.packed || a.col_exp), "concord_materialize_group: NULL argument");
+    CONCORD_CHECK(!a.packed || (a.ld_p >= a.K && a.ld_out >= a.K),
+                  "concord_materialize_group: leading dimension < K");
+  }
+  hipStream_t st = (hipStream_t)stream;
+  Group g{};
+  uint32_t blocks = 0;
+  auto flush = [&] {
+    if (g.n == 0) return;
+    if (consolidated) hipLaunchKernelGGL((materialize_group_kernel<true>), dim3(blocks), dim3(256), 0, st, g);
+    else hipLaunchKernelGGL((materialize_group_kernel<false>), dim3(blocks), dim3(256), 0, st, g);
+    g = Group{};
+    blocks = 0;
+  };
+  for (int32_t i = 0; i < n; ++i) {
+    const concord_materialize_item& a = items[i];
+    if (a.N == 0 || a.K == 0) continue;
+    GroupItem t{};
+    const int64_t cpr = cdiv(a.K, 8), chunks = a.packed ? a.N * cpr : cdiv(a.N, 8);
+    if (chunks >= (1LL << 31)) {   // (more words than the 32-bit chunk count holds)
+      const int rc = concord_materialize(a.packed, a.ld_p, a.row_exp, a.col_exp, a.N, a.K, (int32_t)a.mantissa_bias,
+                                         consolidated, a.out, a.ld_out, stream);
+      if (rc != CONCORD_OK) return rc;
+      continue;
+    }
+    t.packed = a.packed;
+    t.row_exp = a.row_exp;
+    t.col_exp = a.col_exp;
+    t.out = a.out;
+    t.ld_p = a.ld_p;
+    t.ld_o = a.ld_out;
+    t.K = a.K;
+    t.chunks = (uint32_t)chunks;
+    t.cpr = (uint32_t)cpr;
+    t.first = blocks;
+    t.bias = (int32_t)a.mantissa_bias;
+    t.vec = a.packed ? (a.ld_p % 4 == 0 && a.ld_out % 8 == 0 && (uintptr_t)a.packed % 16 == 0 && (uintptr_t)a.out % 16 == 0)
+                     : ((uintptr_t)a.row_exp % 8 == 0 && (uintptr_t)a.out % 8 == 0);
+    t.tail = a.packed ? 0 : (int32_t)(a.N - (chunks - 1) * 8);
+    g.it[g.n++] = t;
+    blocks += (uint32_t)cdiv(chunks, kGroupChunks);
+    if (g.n == kGroupItems || blocks >= (1u << 22)) flush();
+  }
+  flush();
+  return launch_status("materialize_group");
 }
 
 extern "C" int concord_materialize_gated(const int32_t* packed, int64_t ld_p, const int8_t* row_exp,

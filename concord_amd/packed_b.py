@@ -1758,18 +1758,61 @@ def reference_state_dict(module):
             if not (k == '_extra_state' or k.endswith('._extra_state'))}
 
 
+def _consolidated_group(layers):
+    """consolidated_weight() of packed layers of one device and copies of their
+    biases, all in one grouped launch per 24 tensors."""
+    dev = layers[0].packed_w.device
+    fields, ws, bs = [], [], []
+    for m in layers:
+        pw = m.packed_w
+        N, K = _check_packed(pw, m.row_exp, m.col_exp)
+        W = torch.empty((N, K), dtype=torch.bfloat16, device=dev)
+        fields += (pw.data_ptr(), pw.stride(0), m.row_exp.data_ptr(), m.col_exp.data_ptr(), N, K, W.data_ptr(), K,
+                   m.MANTISSA_BIAS)
+        b = getattr(m, 'bias', None)
+        if b is not None:
+            b = b.detach()
+            if b.device == dev and b.is_contiguous():
+                c = torch.empty_like(b)
+                fields += (0, 0, b.data_ptr(), 0, b.numel() * b.element_size(), 1, c.data_ptr(), 0, 0)
+                b = c
+            else:
+                b = b.clone()
+        ws.append(W)
+        bs.append(b)
+    n = len(fields)
+    C.check(C.lib().concord_materialize_group((ctypes.c_int64 * n)(*fields), n // 9, 1, C.stream_of(dev)),
+            "consolidated_state_dict")
+    return ws, bs
+
+
 @torch.no_grad()
 def consolidated_state_dict(layers, names):
     """Deploy export (notebook/src/concord_winner.py:328-341): each layer's
     consolidated_weight() (s_fast dropped) as name + '.weight', its bias as
     name + '.bias'; conv weights as (out, in, kh, kw); plain bf16
     tensors for safetensors / nn.Linear / nn.Conv2d."""
+    pairs = list(zip(names, layers))
+    groups = {}
+    for i, (_, m) in enumerate(pairs):
+        if type(m) in (ConcordLinearPackedB, ConcordConv2dPackedB):   # no override of consolidated_weight
+            groups.setdefault(m.packed_w.device, []).append(i)
+    done = {}
+    for dev, at in groups.items():
+        if dev.type == "cuda":
+            ws, bs = _consolidated_group([pairs[i][1] for i in at])
+            done.update(zip(at, zip(ws, bs)))
     out = {}
-    for name, m in zip(names, layers):
-        W = m.consolidated_weight()
+    for i, (name, m) in enumerate(pairs):
+        if i in done:
+            W, b = done[i]
+        else:
+            W = m.consolidated_weight()
+            b = getattr(m, 'bias', None)
+            b = None if b is None else b.detach().clone()
         if isinstance(m, ConcordConv2dPackedB):
             W = W.view(m.out_channels, m.in_channels, m.kh, m.kw)
         out[name + '.weight'] = W
-        if getattr(m, 'bias', None) is not None:
-            out[name + '.bias'] = m.bias.detach().clone()
+        if b is not None:
+            out[name + '.bias'] = b
     return out

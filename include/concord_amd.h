@@ -92,6 +92,21 @@ int concord_materialize(const int32_t* packed, int64_t ld_p, const int8_t* row_e
                         const int8_t* col_exp, int64_t N, int64_t K, int32_t mantissa_bias,
                         int consolidated, uint16_t* out, int64_t ld_out, void* stream);
 
+/* concord_materialize of n layers (and plain copies: packed NULL, N bytes from
+ * row_exp to out, at most 2^31) in one launch per 24 items; the items are read
+ * before the call returns. */
+typedef struct {
+  const int32_t* packed;
+  int64_t ld_p;
+  const int8_t* row_exp;
+  const int8_t* col_exp;
+  int64_t N, K;
+  uint16_t* out;
+  int64_t ld_out;
+  int64_t mantissa_bias;
+} concord_materialize_item;
+int concord_materialize_group(const concord_materialize_item* items, int32_t n, int consolidated, void* stream);
+
 /* The forward weight with s_fast gated by fast_gain in [0, 1):
  * bf16(((128 s_slow + fast_gain s_fast) + 128 v_slow) * 2^(row_exp + col_exp -
  * mantissa_bias)), fp32 ops in that order.  Replaces the torch re-materialise
