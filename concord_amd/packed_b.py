@@ -19,6 +19,7 @@ Two forward/dgrad modes, both bit-identical in what they feed the MFMAs:
                                 GEMMs read it.
 """
 import ctypes
+import functools
 import math
 
 import torch
@@ -125,11 +126,17 @@ def set_prototype_semantics(enabled):
 # Per-device device scalars (concord/packed_b.py:315-359; prototype 331-353,
 # 1016-1046)
 # ---------------------------------------------------------------------------
+_DEV_KEYS = {}   # device -> key, for devices that name their index
+
+
 def _dev_key(device):
-    d = torch.device(device)
-    if d.type == "cuda" and d.index is None:
-        d = torch.device("cuda", torch.cuda.current_device())
-    return str(d)
+    key = _DEV_KEYS.get(device)
+    if key is None:
+        d = torch.device(device)
+        if d.type == "cuda" and d.index is None:
+            return str(torch.device("cuda", torch.cuda.current_device()))
+        key = _DEV_KEYS[device] = str(d)
+    return key
 
 
 _STEP_COUNTERS = {}
@@ -227,14 +234,27 @@ def _ensure_reb_seed_tensor(device):
 _GEMM_WORKSPACES = {}
 
 
+# the sizes below are functions of the problem alone; a call plans every product
+# of the layer (5 - 20 us), so they are kept per problem
+@functools.lru_cache(maxsize=4096)
+def _gemm_need(M, N, K):
+    L = C.lib()
+    return int(L.concord_gemm_workspace_bytes(M, N, K)), bool(L.concord_gemm_decodes_weight(M, N, K))
+
+
+@functools.lru_cache(maxsize=4096)
+def _need(N, K, M):
+    return int(C.lib().concord_workspace_bytes(N, K, M))
+
+
 def _gemm_workspace(device, M, N, K):
     """Zero-initialised per-device split-K workspace of the GEMMs, grown to the
     largest problem seen (grow it eagerly, before any graph capture).  A layer
     whose products decode the weight into the workspace gets its own from the
     allocator: forwards on several streams must not share it."""
     key = _dev_key(device)
-    need = int(C.lib().concord_gemm_workspace_bytes(int(M), int(N), int(K)))
-    if C.lib().concord_gemm_decodes_weight(int(M), int(N), int(K)):
+    need, decodes = _gemm_need(int(M), int(N), int(K))
+    if decodes:
         return torch.empty(need, dtype=torch.uint8, device=key)
     ws = _GEMM_WORKSPACES.get(key)
     if ws is None or ws.numel() < need:
@@ -246,7 +266,7 @@ def _gemm_workspace(device, M, N, K):
 def _workspace(device, N, K, M=0):
     """Zero-initialised per-device workspace, grown to the largest layer."""
     key = _dev_key(device)
-    need = int(C.lib().concord_workspace_bytes(int(N), int(K), int(M)))
+    need = _need(int(N), int(K), int(M))
     ws = _WORKSPACES.get(key)
     if ws is None or ws.numel() < need:
         ws = torch.zeros(need, dtype=torch.uint8, device=key)
@@ -662,7 +682,7 @@ def muon_ns5(grad_W, out=None, gamma=None):
 
 def _bias_grad(dy):
     M, N = dy.shape
-    need = int(C.lib().concord_workspace_bytes(N, 1, M))
+    need = _need(N, 1, M)
     scratch = torch.empty(need, dtype=torch.uint8, device=dy.device)
     out = torch.empty(N, dtype=torch.bfloat16, device=dy.device)
     C.check(C.lib().concord_bias_grad(C.ptr(dy), dy.stride(0), M, N, C.ptr(out), C.ptr(scratch),
