@@ -77,7 +77,7 @@ struct GemmArgs {
   // i-tiles per group of the grouped tile order (grouped_tile); 0: 8.  The
   // order only decides which workgroup computes which tile, never a result.
   int gi;
-  // pad: the operands are zero-padded copies (ragged.h), readable in whole
+  // pad: the operands are zero-padded copies (gemm.hip), readable in whole
   // chunks of 8 columns past I / J; sc: the output rows allow no 8-byte
   // stores (J or ldc no multiple of 4, or c not 8-byte aligned)
   int pad, sc;

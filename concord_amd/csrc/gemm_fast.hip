@@ -319,7 +319,7 @@ struct ColsBf16 {
     rb = G::rb(t);
     ld2 = (uint32_t)(ld * 2);
     // (cols_left is a multiple of 4, or the operand is padded to one)
-    rs = make_rsrc(band, nrec(((R - 1) * ld + (cols_left + 3) / 4 * 4) * 2));
+    rs = make_rsrc(band, nrec(((R - 1) * ld + ((cols_left + 3) & ~(int64_t)3)) * 2));
 #pragma unroll
     for (int q = 0; q < PER; ++q) {
       const int64_t col = G::col(t, q);
@@ -459,14 +459,13 @@ CONCORD_DEV float* partial_slot(const GemmArgs& g, int tile, int split, int aw) 
 }
 
 // products that may have a ragged output (g.sc): the packed modes do not
-// (their split-K reduction measured 0.4 us longer with the branch)
 template <int MODE>
 constexpr bool ragged_mode() { return MODE != MODE_FWD && MODE != MODE_DGRAD; }
 
-// the bias of columns j .. j + 3 (j < J)
-template <int MODE>
+// the bias of columns j .. j + 3 (j < J); SC: g.sc may be set
+template <bool SC>
 CONCORD_DEV void load_bias4(const GemmArgs& g, int64_t j, float (&bs)[4]) {
-  if (ragged_mode<MODE>() && g.sc) {
+  if (SC && g.sc) {
 #pragma unroll
     for (int e = 0; e < 4; ++e) bs[e] = j + e < g.J ? bf16_to_f32(g.vbias[j + e]) : 0.f;
     return;
@@ -479,10 +478,10 @@ CONCORD_DEV void load_bias4(const GemmArgs& g, int64_t j, float (&bs)[4]) {
 }
 
 // 4 bf16 (o) to columns j .. j + 3 of an output row (j < J)
-template <int MODE>
+template <bool SC>
 CONCORD_DEV void store4(const GemmArgs& g, int64_t i, int64_t j, uint2 o) {
   uint16_t* c = g.c + i * g.ldc + j;
-  if (!ragged_mode<MODE>() || !g.sc) {
+  if (!SC || !g.sc) {
     *reinterpret_cast<uint2*>(c) = o;
     return;
   }
@@ -523,7 +522,7 @@ CONCORD_DEV void epilogue(const GemmArgs& g, f32x4 (&acc)[NI][NJ], int64_t i0, i
 #pragma unroll
           for (int e = 0; e < 4; ++e) sc[e] = exp2i(sbyte(e4, e) - g.bias);
         }
-        if (g.vbias) load_bias4<MODE>(g, j, bs);
+        if (g.vbias) load_bias4<ragged_mode<MODE>()>(g, j, bs);
       }
 #pragma unroll
       for (int x = 0; x < NI; ++x) {
@@ -602,7 +601,7 @@ CONCORD_DEV int64_t splitk_reduce_items(const GemmArgs& g) {
   return tiles * WI * WJ * NI * NJ * 64;
 }
 
-template <int MODE, int NI, int NJ, int BI, int BJ, int WI, int WJ, int SP>
+template <int MODE, int NI, int NJ, int BI, int BJ, int WI, int WJ, int SP, bool SC>
 CONCORD_DEV void splitk_reduce_item_sp(const GemmArgs& g, int64_t idx) {
   constexpr int NAW = WI * WJ, WTI = BI / WI, WTJ = BJ / WJ;
   const int lane = (int)(idx % 64);
@@ -634,7 +633,7 @@ CONCORD_DEV void splitk_reduce_item_sp(const GemmArgs& g, int64_t idx) {
 #pragma unroll
     for (int e = 0; e < 4; ++e) sc[e] = exp2i(sbyte(e4, e) - g.bias);
   }
-  if (g.vbias) load_bias4<MODE>(g, j, bs);
+  if (g.vbias) load_bias4<SC>(g, j, bs);
   float v[4];
 #pragma unroll
   for (int e = 0; e < 4; ++e) v[e] = __fadd_rn(__fmul_rn(sum[e], sc[e]), bs[e]);
@@ -659,29 +658,29 @@ CONCORD_DEV void splitk_reduce_item_sp(const GemmArgs& g, int64_t idx) {
     }
     return;
   }
-  store4<MODE>(g, i, j, o);
+  store4<SC>(g, i, j, o);
 }
 
 // splitk_reduce_item_sp for the launch's split count (uniform), 2 .. kGemmMaxSplits
-template <int MODE, int NI, int NJ, int BI, int BJ, int WI, int WJ>
+template <int MODE, int NI, int NJ, int BI, int BJ, int WI, int WJ, bool SC = false>
 CONCORD_DEV void splitk_reduce_item(const GemmArgs& g, int64_t idx) {
   static_assert(kGemmMaxSplits == 16, "one case per split count");
   switch (g.splits) {
-    case 2: splitk_reduce_item_sp<MODE, NI, NJ, BI, BJ, WI, WJ, 2>(g, idx); break;
-    case 3: splitk_reduce_item_sp<MODE, NI, NJ, BI, BJ, WI, WJ, 3>(g, idx); break;
-    case 4: splitk_reduce_item_sp<MODE, NI, NJ, BI, BJ, WI, WJ, 4>(g, idx); break;
-    case 5: splitk_reduce_item_sp<MODE, NI, NJ, BI, BJ, WI, WJ, 5>(g, idx); break;
-    case 6: splitk_reduce_item_sp<MODE, NI, NJ, BI, BJ, WI, WJ, 6>(g, idx); break;
-    case 7: splitk_reduce_item_sp<MODE, NI, NJ, BI, BJ, WI, WJ, 7>(g, idx); break;
-    case 8: splitk_reduce_item_sp<MODE, NI, NJ, BI, BJ, WI, WJ, 8>(g, idx); break;
-    case 9: splitk_reduce_item_sp<MODE, NI, NJ, BI, BJ, WI, WJ, 9>(g, idx); break;
-    case 10: splitk_reduce_item_sp<MODE, NI, NJ, BI, BJ, WI, WJ, 10>(g, idx); break;
-    case 11: splitk_reduce_item_sp<MODE, NI, NJ, BI, BJ, WI, WJ, 11>(g, idx); break;
-    case 12: splitk_reduce_item_sp<MODE, NI, NJ, BI, BJ, WI, WJ, 12>(g, idx); break;
-    case 13: splitk_reduce_item_sp<MODE, NI, NJ, BI, BJ, WI, WJ, 13>(g, idx); break;
-    case 14: splitk_reduce_item_sp<MODE, NI, NJ, BI, BJ, WI, WJ, 14>(g, idx); break;
-    case 15: splitk_reduce_item_sp<MODE, NI, NJ, BI, BJ, WI, WJ, 15>(g, idx); break;
-    default: splitk_reduce_item_sp<MODE, NI, NJ, BI, BJ, WI, WJ, 16>(g, idx); break;
+    case 2: splitk_reduce_item_sp<MODE, NI, NJ, BI, BJ, WI, WJ, 2, SC>(g, idx); break;
+    case 3: splitk_reduce_item_sp<MODE, NI, NJ, BI, BJ, WI, WJ, 3, SC>(g, idx); break;
+    case 4: splitk_reduce_item_sp<MODE, NI, NJ, BI, BJ, WI, WJ, 4, SC>(g, idx); break;
+    case 5: splitk_reduce_item_sp<MODE, NI, NJ, BI, BJ, WI, WJ, 5, SC>(g, idx); break;
+    case 6: splitk_reduce_item_sp<MODE, NI, NJ, BI, BJ, WI, WJ, 6, SC>(g, idx); break;
+    case 7: splitk_reduce_item_sp<MODE, NI, NJ, BI, BJ, WI, WJ, 7, SC>(g, idx); break;
+    case 8: splitk_reduce_item_sp<MODE, NI, NJ, BI, BJ, WI, WJ, 8, SC>(g, idx); break;
+    case 9: splitk_reduce_item_sp<MODE, NI, NJ, BI, BJ, WI, WJ, 9, SC>(g, idx); break;
+    case 10: splitk_reduce_item_sp<MODE, NI, NJ, BI, BJ, WI, WJ, 10, SC>(g, idx); break;
+    case 11: splitk_reduce_item_sp<MODE, NI, NJ, BI, BJ, WI, WJ, 11, SC>(g, idx); break;
+    case 12: splitk_reduce_item_sp<MODE, NI, NJ, BI, BJ, WI, WJ, 12, SC>(g, idx); break;
+    case 13: splitk_reduce_item_sp<MODE, NI, NJ, BI, BJ, WI, WJ, 13, SC>(g, idx); break;
+    case 14: splitk_reduce_item_sp<MODE, NI, NJ, BI, BJ, WI, WJ, 14, SC>(g, idx); break;
+    case 15: splitk_reduce_item_sp<MODE, NI, NJ, BI, BJ, WI, WJ, 15, SC>(g, idx); break;
+    default: splitk_reduce_item_sp<MODE, NI, NJ, BI, BJ, WI, WJ, 16, SC>(g, idx); break;
   }
 }
 
@@ -698,12 +697,14 @@ CONCORD_DEV void bias_fold_item(const GemmArgs& g, int64_t f) {
 
 // threads [0, items) reduce the product; for a WGRAD with bias partials the
 // next tiles_j * I fold them
-template <int MODE, int NI, int NJ, int BI, int BJ, int WI, int WJ>
+// SC: a ragged output (its own kernel: the check in every item's loads and
+// store cost the packed reductions 0.4 us a launch)
+template <int MODE, int NI, int NJ, int BI, int BJ, int WI, int WJ, bool SC>
 __global__ __launch_bounds__(256) void splitk_reduce_kernel(GemmArgs g) {
   const int64_t idx = (int64_t)blockIdx.x * 256 + threadIdx.x;
   const int64_t items = splitk_reduce_items<MODE, NI, NJ, BI, BJ, WI, WJ>(g);
   if (idx < items) {
-    splitk_reduce_item<MODE, NI, NJ, BI, BJ, WI, WJ>(g, idx);
+    splitk_reduce_item<MODE, NI, NJ, BI, BJ, WI, WJ, SC>(g, idx);
   } else if (MODE == MODE_WGRAD && g.bpart && idx - items < (int64_t)g.tiles_j * g.I) {
     bias_fold_item(g, idx - items);
   }
@@ -773,7 +774,7 @@ struct ReduceVh {
 #pragma unroll
         for (int e = 0; e < 4; ++e) s_g2[((x * NJ + y) * 4 + e) * 64 + lane] = __fmul_rn(v[e], v[e]);
         const int64_t i = row0 + x * 16 + (lane & 15), j = col0 + y * 16 + 4 * (lane >> 4);
-        if (i < g.I && j < g.J) store4<MODE_WGRAD>(g, i, j, make_uint2(lo, hi));
+        if (i < g.I && j < g.J) store4<true>(g, i, j, make_uint2(lo, hi));
       }
     }
     if (x == 1 && g.bpart && aw % WJ == 0) {
@@ -1459,7 +1460,7 @@ struct TrDma {
     lrow = lane / (ROWB / 16);
     const uint64_t base = (uint64_t)(uintptr_t)band;
     // (cols_left is a multiple of 8, or the operand is padded to one)
-    const int64_t bytes = ((R - 1) * ld + (cols_left < COLS ? (cols_left + 7) / 8 * 8 : COLS)) * 2;
+    const int64_t bytes = ((R - 1) * ld + (cols_left < COLS ? ((cols_left + 7) & ~(int64_t)7) : COLS)) * 2;
     rs = i32x4{(int32_t)(uint32_t)base, (int32_t)(uint32_t)((base >> 32) & 0xFFFF), (int32_t)nrec(bytes),
                0x00020000};
     for (int e = 0; e < 4; ++e) rs[e] = __builtin_amdgcn_readfirstlane(rs[e]);
@@ -1831,7 +1832,7 @@ struct TrRowsB {
     rg = t / CG;
     ldb = (uint32_t)(ld * ES);
     // (cols_left is a multiple of 4, or the operand is padded to one)
-    rs = make_rsrc(band, nrec(((R - 1) * ld + (cols_left + 3) / 4 * 4) * ES));
+    rs = make_rsrc(band, nrec(((R - 1) * ld + ((cols_left + 3) & ~(int64_t)3)) * ES));
     if (PACKED) es = make_rsrc(exps, (uint32_t)R);
     voff = col < cols_left ? (uint32_t)((8 * rg * ld + col) * ES) : kOOB;
   }
@@ -2254,8 +2255,13 @@ static void launch_reduce(const GemmArgs& g, hipStream_t st) {
   constexpr int NI = BI / WI / 16, NJ = BJ / WJ / 16;
   int64_t threads = (g.sym ? (int64_t)g.sym : (int64_t)g.tiles_i * g.tiles_j) * WI * WJ * NI * NJ * 64;
   if (MODE == MODE_WGRAD && g.bpart) threads += (int64_t)g.tiles_j * g.I;   // the bias fold
-  hipLaunchKernelGGL((splitk_reduce_kernel<MODE, NI, NJ, BI, BJ, WI, WJ>), dim3((unsigned)cdiv(threads, 256)),
-                     dim3(256), 0, st, g);
+  const dim3 grid((unsigned)cdiv(threads, 256));
+  if constexpr (ragged_mode<MODE>())
+    if (g.sc) {
+      hipLaunchKernelGGL((splitk_reduce_kernel<MODE, NI, NJ, BI, BJ, WI, WJ, true>), grid, dim3(256), 0, st, g);
+      return;
+    }
+  hipLaunchKernelGGL((splitk_reduce_kernel<MODE, NI, NJ, BI, BJ, WI, WJ, false>), grid, dim3(256), 0, st, g);
 }
 
 template <int MODE, int BI, int BJ>
