@@ -491,7 +491,8 @@ CONCORD_DEV void store4(const GemmArgs& g, int64_t i, int64_t j, uint2 o) {
     if (j + e < g.J) c[e] = (uint16_t)(w[e / 2] >> (16 * (e & 1)));
 }
 
-template <int MODE, int NI, int NJ, int BI, int BJ, int NAW>
+// SC: the output may be ragged (g.sc)
+template <int MODE, int NI, int NJ, int BI, int BJ, int NAW, bool SC = ragged_mode<MODE>()>
 CONCORD_DEV void epilogue(const GemmArgs& g, f32x4 (&acc)[NI][NJ], int64_t i0, int64_t j0, int ra, int rb,
                           int split, int tile, int aw, int t, int nthreads, uint16_t* stage) {
   constexpr int LDO = BJ + 8;   // bf16 per staged row (16-byte multiple, shifts banks by 4)
@@ -522,7 +523,7 @@ CONCORD_DEV void epilogue(const GemmArgs& g, f32x4 (&acc)[NI][NJ], int64_t i0, i
 #pragma unroll
           for (int e = 0; e < 4; ++e) sc[e] = exp2i(sbyte(e4, e) - g.bias);
         }
-        if (g.vbias) load_bias4<ragged_mode<MODE>()>(g, j, bs);
+        if (g.vbias) load_bias4<SC>(g, j, bs);
       }
 #pragma unroll
       for (int x = 0; x < NI; ++x) {
@@ -539,7 +540,7 @@ CONCORD_DEV void epilogue(const GemmArgs& g, f32x4 (&acc)[NI][NJ], int64_t i0, i
   // row-contiguous stores: 8 bf16 (16 bytes) per thread when the output
   // allows, else 4 (J % 4 == 0, ldc % 4 == 0, 8-byte aligned base)
   const bool v16 = (g.ldc % 8 == 0) && (g.J % 8 == 0) && (((uintptr_t)g.c % 16) == 0);
-  if (ragged_mode<MODE>() && g.sc) {
+  if (SC && g.sc) {
     // ragged rows: one element per thread, consecutive threads consecutive columns
     for (int c = t; c < BI * BJ; c += nthreads) {
       const int rl = c / BJ, cl = c % BJ;
@@ -1619,7 +1620,7 @@ CONCORD_DEV void bias_acc(f32x4 (&b)[NI], const bf16x8 (&fa)[NI]) {
 // (wgrad_update.h); every workgroup meets the grid barriers, the WGRAD
 // workgroups update their tiles from the accumulators, and the bf16 weight
 // gradient is stored only when g.c is set.
-template <int BI, int BJ, int WI, int WJ, bool VH, bool CONV, int RBI, int UPD>
+template <int BI, int BJ, int WI, int WJ, bool VH, bool CONV, int RBI, int UPD, bool SC>
 CONCORD_DEV void gemm_tr_body(const GemmArgs& g, const GemmArgs& rd, int tr_blocks, const WgradUpd& u, uint32_t wg,
                               uint32_t ngrid, uint16_t* ring_mem, int* s_flag_mem) {
   constexpr int NW = WI * WJ, NT = 64 * NW, WTI = BI / WI, WTJ = BJ / WJ;
@@ -1763,7 +1764,7 @@ CONCORD_DEV void gemm_tr_body(const GemmArgs& g, const GemmArgs& rd, int tr_bloc
     vhat_tile_partials<UPD != 0>(g2, lane, i0 + wi * WTI, j0 + wj * WTJ, g.I, g.J, g.vh_pr, g.vh_pc);
   }
   if (UPD == 0 || g.c)
-    epilogue<MODE_WGRAD, NI, NJ, BI, BJ, NW>(g, acc, i0, j0, wi * WTI, wj * WTJ, split, bi * g.tiles_j + bj, wave, t,
+    epilogue<MODE_WGRAD, NI, NJ, BI, BJ, NW, SC>(g, acc, i0, j0, wi * WTI, wj * WTJ, split, bi * g.tiles_j + bj, wave, t,
                                              NT, ring);
   if constexpr (UPD != 0) {
     const bool bad = grid_sync(u, ngrid, &s_flag);
@@ -1787,7 +1788,7 @@ constexpr int tr_ring_bytes() { return 3 * (TR * BI * 2 + TR * BJ * 2); }
 template <int BI, int BJ, int WI, int WJ, bool VH, bool CONV = false, int RBI = 256>
 __global__ __launch_bounds__(64 * WI * WJ, 1) void gemm_tr_kernel(GemmArgs g, GemmArgs rd, int tr_blocks) {
   __shared__ __attribute__((aligned(1024))) char lds[tr_ring_bytes<BI, BJ>() + 16];
-  gemm_tr_body<BI, BJ, WI, WJ, VH, CONV, RBI, 0>(g, rd, tr_blocks, WgradUpd{}, blockIdx.x, gridDim.x,
+  gemm_tr_body<BI, BJ, WI, WJ, VH, CONV, RBI, 0, !CONV>(g, rd, tr_blocks, WgradUpd{}, blockIdx.x, gridDim.x,
                                                  reinterpret_cast<uint16_t*>(lds),
                                                  reinterpret_cast<int*>(lds + tr_ring_bytes<BI, BJ>()));
 }
@@ -1797,7 +1798,7 @@ __global__ __launch_bounds__(64 * WI * WJ, 1) void gemm_tr_kernel(GemmArgs g, Ge
 template <int RBI, int UPD>
 __global__ __launch_bounds__(512, 1) void wgrad_update_kernel(GemmArgs g, GemmArgs rd, int tr_blocks, WgradUpd u) {
   __shared__ __attribute__((aligned(1024))) char lds[tr_ring_bytes<256, 128>() + 16];
-  gemm_tr_body<256, 128, 4, 2, true, false, RBI, UPD>(g, rd, tr_blocks, u, blockIdx.x, gridDim.x,
+  gemm_tr_body<256, 128, 4, 2, true, false, RBI, UPD, false>(g, rd, tr_blocks, u, blockIdx.x, gridDim.x,
                                                       reinterpret_cast<uint16_t*>(lds),
                                                       reinterpret_cast<int*>(lds + tr_ring_bytes<256, 128>()));
 }
@@ -2068,7 +2069,7 @@ __global__ __launch_bounds__(512, 1) void gemm_dgt_tr_kernel(GemmArgs gd, GemmAr
                                                   lds + A);
   } else {
     const int tw = (int)gridDim.x - dg_blocks;   // every remaining workgroup has a tile: no carried blocks
-    gemm_tr_body<256, 128, 4, 2, true, false, 256, 0>(gw, gw, tw, WgradUpd{}, (uint32_t)(wg - dg_blocks),
+    gemm_tr_body<256, 128, 4, 2, true, false, 256, 0, false>(gw, gw, tw, WgradUpd{}, (uint32_t)(wg - dg_blocks),
                                                       (uint32_t)tw, reinterpret_cast<uint16_t*>(lds),
                                                       reinterpret_cast<int*>(lds + T));
   }
