@@ -81,6 +81,8 @@ struct GemmArgs {
   // chunks of 8 columns past I / J; sc: the output rows allow no 8-byte
   // stores (J or ldc no multiple of 4, or c not 8-byte aligned)
   int pad, sc;
+  // > 0: the split count the bf16 kernels take, where their workspace holds it
+  int keep;
 };
 
 // s * y + t * x as the Newton-Schulz combination steps take it (x is the
@@ -266,10 +268,13 @@ int gemm_conv_launch(int mode, const GemmArgs& g, void* workspace, size_t ws_byt
 size_t gemm_conv_partial_bytes(int mode, int64_t I, int64_t J, int64_t R);
 // split-K workspace bytes (counters + partials) one such product may use
 size_t gemm_splitk_need(int mode, int64_t I, int64_t J, int64_t R);
-// split-K partial bytes the fast kernels plan for an I x J x R problem
-// given unlimited workspace (0 when they do not split it)
+// workspace bytes gemm_bf16_run (MODE_FWD_BF16, MODE_DGRAD_BF16) may use: the
+// above, and the padded copies of ragged operands
+size_t gemm_bf16_need(int mode, int64_t I, int64_t J, int64_t R);
 // the packed product (MODE_FWD, MODE_DGRAD) runs on a decoded copy of its weight
 bool gemm_decode_pays(int mode, int64_t I, int64_t J, int64_t R);
-size_t gemm_fast_partial_bytes(int mode, int64_t I, int64_t J, int64_t R);
+// split-K partial bytes the fast kernels plan for an I x J x R problem given
+// unlimited workspace (0 when they do not split it); keep as in GemmArgs
+size_t gemm_fast_partial_bytes(int mode, int64_t I, int64_t J, int64_t R, int keep = 0);
 
 }  // namespace concord

@@ -701,6 +701,9 @@ int gemm_bf16_run(int mode, const uint16_t* a, int64_t lda, const uint16_t* b, i
                   int64_t ldc, int64_t I, int64_t J, int64_t R, void* ws, size_t ws_bytes, hipStream_t st,
                   const char* what) {
   GemmArgs g = make_args(a, b, lda, ldb, nullptr, nullptr, 0, nullptr, c, ldc, I, J, R, false);
+  // operands the fast kernels take only as padded copies: the sums of the
+  // generic kernel (its two ways at most), so the copies change no bit
+  if (mode != MODE_WGRAD && !gemm_fast_takes(mode, g)) g.keep = plan_gemm(I, J, R, true).splits;
   if (mode == MODE_FWD_BF16) return launch_gemm<MODE_FWD_BF16>(g, ws, ws_bytes, st, what);
   if (mode == MODE_DGRAD_BF16) return launch_gemm<MODE_DGRAD_BF16>(g, ws, ws_bytes, st, what);
   if (mode == MODE_WGRAD) return launch_gemm<MODE_WGRAD>(g, ws, ws_bytes, st, what);
@@ -723,6 +726,15 @@ int gemm_bf16_combine(int mode, const uint16_t* a, int64_t lda, const uint16_t* 
 
 size_t gemm_splitk_need(int mode, int64_t I, int64_t J, int64_t R) {
   return kSplitkCounterBytes + ((splitk_partials(mode, I, J, R) + 255) / 256) * 256;
+}
+
+size_t gemm_bf16_need(int mode, int64_t I, int64_t J, int64_t R) {
+  const bool fwd = mode == MODE_FWD_BF16;
+  const size_t plain = gemm_splitk_need(mode, I, J, R);
+  const RaggedRoom r = fwd ? ragged_room(I, J, R) : ragged_room(I, R, J);
+  if (r.total == 0) return plain;
+  const size_t part = gemm_fast_partial_bytes(mode, I, J, R, plan_gemm(I, J, R, true).splits);
+  return std::max(plain, kSplitkCounterBytes + round256(part) + r.total + 256);
 }
 
 }  // namespace concord

@@ -2164,28 +2164,25 @@ static FastPlan plan(const FastShape (&shapes)[NS], int64_t I, int64_t J, int64_
 // 1280 took 102.7, 110.2, 122.8 and 105.6 us in 256 x 256, 256 x 128, 192 x 128
 // and 256 x 160 tiles, 2048 x 1280 x 5120 94.9, 48.3, 42.9, 64.6 unsplit and
 // 40.0, 34.8, 34.7, 36.7 at its best split.
-struct DdShape { int bi, bj, waves; double stage, full; };   // full: the fixed part's growth on a full chip
-constexpr DdShape kDdShapes[] = {{256, 160, 4, 0.74, 4.0}, {256, 256, 8, 1.165, 4.0}, {256, 128, 8, 0.545, 4.0},
-                                 {192, 128, 4, 0.477, 2.0}, {128, 128, 4, 0.33, 1.5}};
+struct DdShape { int bi, bj; double stage, full; };   // full: the fixed part's growth on a full chip
+constexpr DdShape kDdShapes[] = {{256, 160, 0.74, 4.0}, {256, 256, 1.165, 4.0}, {256, 128, 0.545, 4.0},
+                                 {192, 128, 0.477, 2.0}, {128, 128, 0.33, 1.5}};
 constexpr int kDdCount = 5;
 
-// fwd: the 256 x 160 tile as well (the dgrad's weight tile has 2^n columns).
-// fixed: the split count, 0 to choose it.
-static FastPlan plan_dd(bool fwd, int64_t I, int64_t J, int64_t R, size_t room, bool sym, int fixed) {
+// The tile shape of a product in `splits` ways (fewer where `room` does not
+// hold their partials).  fwd: the 256 x 160 tile as well (the dgrad's weight
+// tile has 2^n columns).
+static FastPlan plan_dd(bool fwd, int64_t I, int64_t J, int64_t R, size_t room, bool sym, int splits) {
   FastPlan best{kDdCount - 1, 1, 0, 0, R};
   double best_cost = 1e300;
-  for (int s = fwd ? 0 : 1; s < kDdCount; ++s) {
-    const DdShape& sh = kDdShapes[s];
-    const int64_t ti = cdiv(I, sh.bi), tj = cdiv(J, sh.bj);
-    const int64_t tiles = sym ? sym_tile_count((int)ti, (int)tj, sh.bi, sh.bj) : ti * tj;
-    const double area = (double)sh.bi * sh.bj;
-    const size_t slot = (size_t)(tiles * area) * sizeof(float);
-    const int max_splits = (int)std::min<size_t>(kMaxSplits, std::max<size_t>(1, room / slot));
-    for (int sp = fixed ? fixed : 1; sp <= (fixed ? fixed : max_splits); ++sp) {
-      if (sp > max_splits) break;
-      if (!fixed && sp > 1 && (!gemm_splitk_fits(tiles) || tiles >= kCUs)) break;
-      const int64_t rs = cdiv(cdiv(R, sp), TR) * TR;
-      if (sp > 1 && (sp - 1) * rs >= R) break;
+  for (int sp = splits; sp >= 1 && best.ti == 0; --sp) {
+    const int64_t rs = cdiv(cdiv(R, sp), TR) * TR;
+    if (sp > 1 && (sp - 1) * rs >= R) continue;
+    for (int s = fwd ? 0 : 1; s < kDdCount; ++s) {
+      const DdShape& sh = kDdShapes[s];
+      const int64_t ti = cdiv(I, sh.bi), tj = cdiv(J, sh.bj);
+      const int64_t tiles = sym ? sym_tile_count((int)ti, (int)tj, sh.bi, sh.bj) : ti * tj;
+      if (sp > 1 && room / sizeof(float) / sh.bi / sh.bj < (size_t)(tiles * sp)) continue;
       const double stages = (double)cdiv(rs, TR);
       auto round = [&](double fill) {
         return 4.5 + fill * sh.full + stages * sh.stage * (1.0 + 0.2 * fill);
@@ -2193,10 +2190,11 @@ static FastPlan plan_dd(bool fwd, int64_t I, int64_t J, int64_t R, size_t room, 
       const int64_t blocks = tiles * sp, rest = blocks % kCUs;
       double cost = (double)(blocks / kCUs) * round(1.0) + (rest ? round((double)rest / kCUs) : 0.0);
       // an unsplit symmetric product's mirrored 2-byte stores (A A, 1280 x 1280
-      // in 128 x 128 tiles: 37 us unsplit, 13 + 5 us split and reduced)
-      if (sym && sp == 1) cost += std::ceil((double)tiles / kCUs) * area * 1.4e-3;
-      // the partials' write and reduction (a symmetric product stores twice)
-      if (sp > 1) cost += 3.0 + (double)sp * (sym ? (double)tiles * area * 2.2e-6 : (double)I * J * 1.4e-6);
+      // in 128 x 128 tiles: 37 us unsplit, 13 + 5 us split and reduced), and a
+      // split one's partials, computed tiles only
+      if (sym)
+        cost += sp == 1 ? std::ceil((double)tiles / kCUs) * sh.bi * sh.bj * 1.4e-3
+                        : (double)sp * tiles * sh.bi * sh.bj * 2.2e-6;
       if (cost < best_cost * 0.999) {
         best_cost = cost;
         best = FastPlan{s, sp, (int)ti, (int)tj, rs};
@@ -2361,12 +2359,9 @@ static int plan_gi(int mode, const FastPlan& p, int BI, int BJ) {
   return choose_gi(p.ti, p.tj, p.splits, BI * band_bytes_a(mode), BJ * band_bytes_b(mode));
 }
 
-// sym_part_cost: the split-K partial cost of a symmetric product run by the
-// dgrad kernel, measured rather than modelled: NS5's A A (1280 x 1280 x 1280,
-// 40 upper-triangle tiles of 192 x 128) ran 382.5 us per drive with 3 splits
-// against 389.8 us with the 4 the plain coefficient picks (and 384.4 with 2);
-// the forward kernel's X X^T keeps the plain coefficient (6 splits, best of
-// 4, 5, 6 and 8 in the same sweep)
+// sym_part_cost: the split-K partial cost of a symmetric product of the dgrad
+// form.  The split counts that follow from it are part of the Muon drive's
+// results (below): A A of 1280 x 1280 takes 3 splits, X X^T of 1280 x 5120 takes 6.
 static FastPlan plan_mode(int mode, int64_t I, int64_t J, int64_t R, size_t room, bool sym = false) {
   if (mode == MODE_FWD || mode == MODE_FWD_BF16) return plan(kFwdShapes, I, J, R, room, sym);
   if (mode == MODE_WGRAD) return plan(kWgrShapes, I, J, R, room);
@@ -2385,27 +2380,31 @@ static bool dd_takes(int mode, const GemmArgs& g) {
          (mode == MODE_DGRAD_BF16 && g.ldb % 8 == 0 && al(g.b, 16) && (g.pad || g.J % 8 == 0));
 }
 
-// A layer's product on its decoded weight keeps the splits of the product on
-// the packed weight (the same sums in the same order, so the same bits);
-// symmetric and combined products have no such twin.
-static FastPlan dd_plan(int mode, int64_t I, int64_t J, int64_t R, size_t room, bool sym, bool own) {
+// The split count orders a product's fp32 sums, so it is a rule of the problem
+// and not of the kernel that runs it: a layer's product on its decoded weight
+// has the bits of the product on the packed weight, and the Muon drive, whose
+// fifteen rounded products carry every difference on, keeps its result (with
+// counts chosen for these kernels a drive of 1280 x 5120 took 303 us instead of
+// 319 and differed by 0.7%).  keep: the count a caller asks for (0: the rule).
+static FastPlan dd_plan(int mode, int64_t I, int64_t J, int64_t R, size_t room, bool sym, int keep = 0) {
   const bool fwd = mode == MODE_FWD_BF16;
-  const int fixed = own ? 0 : plan_mode(fwd ? MODE_FWD : MODE_DGRAD, I, J, R, room).splits;
-  const FastPlan p = plan_dd(fwd, I, J, R, room, sym, fixed);
-  return p.ti ? p : plan_dd(fwd, I, J, R, room, sym, 0);   // (no room for the fixed splits' partials)
+  const int splits = keep ? keep : plan_mode(fwd ? MODE_FWD : MODE_DGRAD, I, J, R, room, sym).splits;
+  return plan_dd(fwd, I, J, R, room, sym, splits);
+}
+
+static size_t dd_partial_bytes(const FastPlan& p, bool sym) {
+  const DdShape& sh = kDdShapes[p.shape];
+  const size_t tiles = sym ? sym_tile_count(p.ti, p.tj, sh.bi, sh.bj) : (size_t)p.ti * p.tj;
+  return p.splits > 1 ? tiles * sh.bi * sh.bj * sizeof(float) * p.splits : 0;
 }
 
 }  // namespace
 
-size_t gemm_fast_partial_bytes(int mode, int64_t I, int64_t J, int64_t R) {
+size_t gemm_fast_partial_bytes(int mode, int64_t I, int64_t J, int64_t R, int keep) {
   if (I <= 0 || J <= 0) return 0;
   size_t bytes = 0;
   if (mode == MODE_FWD_BF16 || mode == MODE_DGRAD_BF16)
-    for (bool own : {false, true}) {
-      const FastPlan p = dd_plan(mode, I, J, R, (size_t)-1 / 2, false, own);
-      const DdShape& sh = kDdShapes[p.shape];
-      if (p.splits > 1) bytes = std::max(bytes, (size_t)p.ti * p.tj * sh.bi * sh.bj * sizeof(float) * p.splits);
-    }
+    bytes = dd_partial_bytes(dd_plan(mode, I, J, R, (size_t)-1 / 2, false, keep), false);
   if (mode == MODE_FWD_BF16) return bytes;
   const FastPlan p = plan_mode(mode, I, J, R, (size_t)-1 / 2);
   if (p.splits <= 1) return bytes;
@@ -2765,7 +2764,7 @@ static int dd_launch(int mode, const GemmArgs& g0, void* workspace, size_t room,
                      bool sym) {
   GemmArgs g = g0;
   const bool fwd = mode == MODE_FWD_BF16;
-  const FastPlan p = dd_plan(mode, g.I, g.J, g.R, room, sym, sym || g.ay);
+  const FastPlan p = dd_plan(mode, g.I, g.J, g.R, room, sym, g.keep);
   const DdShape& sh = kDdShapes[p.shape];
   g.splits = p.splits;
   g.r_split = p.r_split;
@@ -2875,11 +2874,12 @@ int gemm_bf16_sym(int mode, const uint16_t* a, int64_t lda, const uint16_t* b, i
 
 size_t gemm_sym_splitk_need(int mode, int64_t I, int64_t R) {
   if (I <= 0) return kSplitkCounterBytes;
+  // the bf16 kernels, and the kernels of dgrad operands without 16-byte chunks
+  size_t part = dd_partial_bytes(dd_plan(mode, I, I, R, (size_t)-1 / 2, true), true);
   const FastPlan p = plan_mode(mode, I, I, R, (size_t)-1 / 2, true);
-  size_t part = 0;
-  if (p.splits > 1) {
+  if (mode == MODE_DGRAD_BF16 && p.splits > 1) {
     const FastShape& sh = shape_of(mode, p.shape);
-    part = (size_t)sym_tile_count(p.ti, p.tj, sh.bi, sh.bj) * sh.bi * sh.bj * sizeof(float) * p.splits;
+    part = std::max(part, (size_t)sym_tile_count(p.ti, p.tj, sh.bi, sh.bj) * sh.bi * sh.bj * sizeof(float) * p.splits);
   }
   return kSplitkCounterBytes + ((part + 255) / 256) * 256;
 }

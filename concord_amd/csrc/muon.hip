@@ -254,8 +254,8 @@ static MuonLayout muon_layout(int64_t N, int64_t K) {
   // split-K region of the three products first: its tile counters sit at
   // the workspace's start for every shape, so the zero state each product
   // leaves them in holds across calls of different shapes
-  size_t g = gemm_splitk_need(MODE_FWD_BF16, m, m, n);
-  const size_t g2 = gemm_splitk_need(MODE_DGRAD_BF16, m, m, m), g3 = gemm_splitk_need(MODE_DGRAD_BF16, m, n, m);
+  size_t g = gemm_bf16_need(MODE_FWD_BF16, m, m, n);
+  const size_t g2 = gemm_bf16_need(MODE_DGRAD_BF16, m, m, m), g3 = gemm_bf16_need(MODE_DGRAD_BF16, m, n, m);
   const size_t g4 = gemm_sym_splitk_need(MODE_FWD_BF16, m, n), g5 = gemm_sym_splitk_need(MODE_DGRAD_BF16, m, m);
   for (size_t v : {g2, g3, g4, g5})
     if (v > g) g = v;
