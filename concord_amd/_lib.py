@@ -77,6 +77,7 @@ _SIGS = {
     "concord_load_weights": (ctypes.c_int, [_P, _I, _I, _I, _i, _i, _i, ctypes.c_int, _P, _I, _P,
                                             _P, _P]),
     "concord_gemm_workspace_bytes": (_Z, [_I, _I, _I]),
+    "concord_gemm_workspace_need": (_Z, [_I, _I, _I, ctypes.c_int, _P]),
     "concord_gemm_decodes_weight": (ctypes.c_int, [_I, _I, _I]),
     "concord_dqgemm_fwd": (ctypes.c_int, [_P, _I, _P, _I, _P, _P, _i, _P, _P, _I, _I, _I, _I, _P, _Z,
                                           _P]),

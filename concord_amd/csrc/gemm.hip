@@ -608,6 +608,18 @@ static bool decoded(int mode, const GemmArgs& g, void* workspace, size_t ws_byte
   return true;
 }
 
+// Layers whose calls write operands (padded copies, a decoded weight) into the
+// workspace: their caller gives each call a workspace of its own, and need not
+// clear it.
+static bool own_workspace(int64_t M, int64_t N, int64_t K, bool packed) {
+  return ragged_room(M, N, K).total != 0 || (packed && decode_room(M, N, K) != 0);
+}
+
+__global__ __launch_bounds__(256) void clear_counters_kernel(uint32_t* c, int n) {
+  const int i = blockIdx.x * 256 + threadIdx.x;
+  if (i < n) c[i] = 0u;
+}
+
 template <int MODE>
 static int launch_gemm(GemmArgs g, void* workspace, size_t ws_bytes, hipStream_t st,
                        const char* what) {
@@ -638,12 +650,7 @@ static int launch_gemm(GemmArgs g, void* workspace, size_t ws_bytes, hipStream_t
   }
   const int fast = gemm_fast_launch(MODE, g, workspace, ws_bytes, st, what);
   if (fast != -1) return fast;
-  // the tile counters of a split launch start at zero; a layer with a decoded
-  // weight may pass a fresh workspace
-  const bool can_split = workspace != nullptr &&
-                         (MODE == MODE_WGRAD            ? decode_room(g.R, g.I, g.J)
-                          : MODE == MODE_FWD || MODE == MODE_FWD_BF16 ? decode_room(g.I, g.J, g.R)
-                                                        : decode_room(g.I, g.R, g.J)) == 0;
+  const bool can_split = workspace != nullptr;
   Plan p = plan_gemm(g.I, g.J, g.R, can_split);
   if (p.splits == 2 &&
       (ws_bytes < gemm_splitk_bytes(g.I, g.J) || !gemm_splitk_fits((int64_t)p.ti * p.tj)))
@@ -656,6 +663,14 @@ static int launch_gemm(GemmArgs g, void* workspace, size_t ws_bytes, hipStream_t
     char* base = (char*)workspace;
     g.tile_cnt = (uint32_t*)base;
     g.part = (float*)(base + kSplitkCounterBytes);
+    // a workspace of the call's own may hold anything where the counters are
+    constexpr bool FWD = MODE == MODE_FWD || MODE == MODE_FWD_BF16;
+    const bool own = MODE == MODE_WGRAD ? own_workspace(g.R, g.I, g.J, true)
+                     : FWD              ? own_workspace(g.I, g.J, g.R, MODE == MODE_FWD)
+                                        : own_workspace(g.I, g.R, g.J, MODE == MODE_DGRAD);
+    if (own)
+      hipLaunchKernelGGL(clear_counters_kernel, dim3((unsigned)cdiv(p.ti * p.tj, 256)), dim3(256), 0, st, g.tile_cnt,
+                         p.ti * p.tj);
   }
   const dim3 grid((unsigned)((int64_t)p.ti * p.tj * p.splits)), block(256);
   switch (p.shape) {
@@ -739,7 +754,8 @@ size_t gemm_bf16_need(int mode, int64_t I, int64_t J, int64_t R) {
 
 }  // namespace concord
 
-extern "C" size_t concord_gemm_workspace_bytes(int64_t M, int64_t N, int64_t K) {
+extern "C" size_t concord_gemm_workspace_need(int64_t M, int64_t N, int64_t K, int packed, int* own) {
+  if (own) *own = M > 0 && N > 0 && K > 0 && own_workspace(M, N, K, packed != 0);
   // tile counters + the split-K partials of the largest need among the layer's
   // three products: y [M,N] (reduce K), dx [M,K] (reduce N), gw [N,K] (reduce M)
   if (M < 1) M = 1;
@@ -757,8 +773,12 @@ extern "C" size_t concord_gemm_workspace_bytes(int64_t M, int64_t N, int64_t K) 
       if (v > m) m = v;
     m = round256(m) + r.total + 256;
   }
-  if (const size_t w = decode_room(M, N, K)) m = round256(m) + w + 256;
+  if (const size_t w = packed ? decode_room(M, N, K) : 0) m = round256(m) + w + 256;
   return kSplitkCounterBytes + ((m + 255) / 256) * 256;
+}
+
+extern "C" size_t concord_gemm_workspace_bytes(int64_t M, int64_t N, int64_t K) {
+  return concord_gemm_workspace_need(M, N, K, 1, nullptr);
 }
 
 extern "C" int concord_gemm_decodes_weight(int64_t M, int64_t N, int64_t K) {

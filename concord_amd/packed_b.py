@@ -238,8 +238,9 @@ _GEMM_WORKSPACES = {}
 # of the layer (5 - 20 us), so they are kept per problem
 @functools.lru_cache(maxsize=4096)
 def _gemm_need(M, N, K):
-    L = C.lib()
-    return int(L.concord_gemm_workspace_bytes(M, N, K)), bool(L.concord_gemm_decodes_weight(M, N, K))
+    own = ctypes.c_int(0)
+    need = C.lib().concord_gemm_workspace_need(M, N, K, 1, ctypes.byref(own))
+    return int(need), bool(own.value)
 
 
 @functools.lru_cache(maxsize=4096)
@@ -249,12 +250,13 @@ def _need(N, K, M):
 
 def _gemm_workspace(device, M, N, K):
     """Zero-initialised per-device split-K workspace of the GEMMs, grown to the
-    largest problem seen (grow it eagerly, before any graph capture).  A layer
-    whose products decode the weight into the workspace gets its own from the
-    allocator: forwards on several streams must not share it."""
+    largest problem seen (grow it eagerly, before any graph capture).  A call
+    that writes operands into its workspace (padded copies of a ragged layer's,
+    a decoded weight) gets one of its own from the allocator: forwards on
+    several streams, or in a graph beside eager ones, must not share it."""
     key = _dev_key(device)
-    need, decodes = _gemm_need(int(M), int(N), int(K))
-    if decodes:
+    need, own = _gemm_need(int(M), int(N), int(K))
+    if own:
         return torch.empty(need, dtype=torch.uint8, device=key)
     ws = _GEMM_WORKSPACES.get(key)
     if ws is None or ws.numel() < need:

@@ -226,6 +226,12 @@ int concord_load_weights(const float* W, int64_t ld_w, int64_t N, int64_t K, int
  * 2-way along the reduction and the halves are added in a fixed way
  * (bit-identical whichever half finishes first). */
 size_t concord_gemm_workspace_bytes(int64_t M, int64_t N, int64_t K);
+/* The same for the products of a packed weight, or (packed 0) of a bf16 weight
+ * and the weight gradient alone, which decode nothing.  *own (own may be NULL):
+ * 1 where the calls write operands into the workspace, zero-padded copies or
+ * the decoded weight.  Such a call takes a workspace no other call uses at the
+ * same time, split or not; it need not be zero-filled. */
+size_t concord_gemm_workspace_need(int64_t M, int64_t N, int64_t K, int packed, int* own);
 /* 1 where the layer's large products decode the packed weight once into the
  * workspace (its last bytes) instead of in every tile.  Such a layer's calls
  * need no zero-filled workspace, and may each take a fresh one. */

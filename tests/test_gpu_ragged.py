@@ -116,3 +116,52 @@ def test_ragged_strided_and_small_workspace(oracle, M, N, K):
         assert (y[:, N:] == 7.0).all()
         err = (y[:, :N].double() - base).norm() / base.norm()
         assert err.item() < 2.0 ** -8
+
+
+def test_ragged_forwards_on_two_streams():
+    """Forwards of two ragged layers in flight on two streams, one of them
+    replayed from a graph, give what each gives alone."""
+    import concord_amd as ca
+    torch.manual_seed(1)
+    layers = [ca.ConcordLinearPackedB(k, n, bias=True, device=DEV) for n, k in ((320, 36), (257, 645))]
+    xs = [torch.randn(m, k, device=DEV).to(torch.bfloat16) for m, k in ((32768, 36), (4096, 645))]
+    with torch.no_grad():
+        alone = [la(x).clone() for la, x in zip(layers, xs)]
+        graph = torch.cuda.CUDAGraph()
+        with torch.cuda.graph(graph):
+            captured = layers[0](xs[0])
+        sync()
+        streams = [torch.cuda.Stream() for _ in range(2)]
+        for _ in range(20):
+            with torch.cuda.stream(streams[0]):
+                graph.replay()
+                got = captured.clone()
+            with torch.cuda.stream(streams[1]):
+                ys = [layers[1](xs[1]) for _ in range(4)]
+            sync()
+            assert torch.equal(got, alone[0])
+            for y in ys:
+                assert torch.equal(y, alone[1])
+
+
+@pytest.mark.parametrize("M,N,K", [(4096, 1280, 1280), (16384, 640, 640)])
+def test_split_counters_of_an_uncleared_workspace(M, N, K):
+    """A layer with a workspace of its own whose operands only the generic
+    kernel takes (an odd base): its two-way split, from uncleared memory."""
+    from concord_amd import _lib as C, packed_b as pb
+    gen = torch.Generator().manual_seed(N)
+    dy = torch.randn(M, N, generator=gen).to(torch.bfloat16).to(DEV)
+    x = torch.empty(M * K + 1, dtype=torch.bfloat16, device=DEV)[1:].view(M, K)
+    x.copy_(torch.randn(M, K, generator=gen))
+    need = int(C.lib().concord_gemm_workspace_bytes(M, N, K))
+    outs = []
+    for fill in (0, 0xA5):
+        ws = torch.full((need,), fill, dtype=torch.uint8, device=DEV)
+        gw = torch.empty(N, K, dtype=torch.bfloat16, device=DEV)
+        C.check(C.lib().concord_wgrad(C.ptr(dy), N, C.ptr(x), K, C.ptr(gw), K, M, N, K, C.ptr(ws), need,
+                                      C.stream_of(torch.device(DEV))), "wgrad")
+        outs.append(gw)
+    sync()
+    assert torch.equal(*outs)
+    ref = dy.double().T @ x.double()
+    assert ((outs[0].double() - ref).norm() / ref.norm()).item() < 2.0 ** -8

@@ -219,3 +219,18 @@ def test_rebalance_group_rejects_bad_plans(L):
     ws = ctypes.create_string_buffer(16)
     assert L.concord_rebalance_group(plan, n, ws, 24000, None, ws, 16, 100, None) == C.EWORKSPACE
     assert L.concord_rebalance_group(plan, n, None, 24000, None, ws, 16, 4, None) == C.EINVAL
+
+
+def test_calls_that_write_operands_get_a_workspace_of_their_own(L):
+    """Padded copies of a ragged layer's operands and decoded weights go into the
+    workspace: two such calls in flight (two streams, a graph beside eager
+    calls) must not hold the same buffer."""
+    from concord_amd import packed_b as pb
+    for M, N, K in [(2048, 320, 36), (512, 65, 384), (4096, 1280, 1280)]:
+        a, b = (pb._gemm_workspace("cpu", M, N, K) for _ in range(2))
+        assert a.numel() == b.numel() >= L.concord_gemm_workspace_bytes(M, N, K)
+        assert a.data_ptr() != b.data_ptr(), (M, N, K)
+    # nothing is copied: the zeroed buffer of the device, its tile counters in use
+    for M, N, K in [(308, 1280, 2048), (3, 5, 7)]:
+        assert pb._gemm_workspace("cpu", M, N, K) is pb._gemm_workspace("cpu", M, N, K)
+    pb._GEMM_WORKSPACES.pop("cpu")
