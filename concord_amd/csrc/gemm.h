@@ -268,8 +268,8 @@ int gemm_conv_launch(int mode, const GemmArgs& g, void* workspace, size_t ws_byt
 size_t gemm_conv_partial_bytes(int mode, int64_t I, int64_t J, int64_t R);
 // split-K workspace bytes (counters + partials) one such product may use
 size_t gemm_splitk_need(int mode, int64_t I, int64_t J, int64_t R);
-// workspace bytes gemm_bf16_run (MODE_FWD_BF16, MODE_DGRAD_BF16) may use: the
-// above, and the padded copies of ragged operands
+// workspace bytes gemm_bf16_run may use: the above, and the padded copies of
+// ragged operands
 size_t gemm_bf16_need(int mode, int64_t I, int64_t J, int64_t R);
 // the packed product (MODE_FWD, MODE_DGRAD) runs on a decoded copy of its weight
 bool gemm_decode_pays(int mode, int64_t I, int64_t J, int64_t R);

@@ -461,15 +461,24 @@ constexpr double kRaggedWork = 4096;   // M N K from which the copies are made a
 static int64_t ceil8(int64_t v) { return (v + 7) / 8 * 8; }
 static size_t round256(size_t b) { return (b + 255) / 256 * 256; }
 
-// bytes of the padded copies of a layer's x, dy and weight (0: all of its
-// widths are multiples of 8, or the layer is tiny)
-struct RaggedRoom { size_t x, dy, w, total; };
-static RaggedRoom ragged_room(int64_t M, int64_t N, int64_t K) {
-  RaggedRoom r{0, 0, 0, 0};
+// The padded copies of a layer's x, dy and weight that `products` (bits kFwd,
+// kDgrad, kWgrad) make: their bytes, 0 for an operand used as it is, and the
+// products that run on copies at all: not those with a copy beyond the extents
+// of the fast kernels (fits31), such as the 1.6 GB dy of 16384 rows of a
+// 50257-word head.
+enum { kFwd = 1, kDgrad = 2, kWgrad = 4 };
+struct RaggedRoom { int products; size_t x, dy, w, total; };
+static RaggedRoom ragged_room(int64_t M, int64_t N, int64_t K, int products = kFwd | kDgrad | kWgrad) {
+  RaggedRoom r{0, 0, 0, 0, 0};
   if ((double)M * (double)N * (double)K < kRaggedWork || (N % 8 == 0 && K % 8 == 0)) return r;
-  r.x = round256((size_t)M * ceil8(K) * 2);
-  r.dy = round256((size_t)M * ceil8(N) * 2);
-  r.w = round256((size_t)ceil8(N) * ceil8(K) * 2);
+  auto fits = [](int64_t rows, int64_t cols) { return rows < (1LL << 29) / ceil8(cols); };
+  const bool x = fits(M, K), dy = fits(M, N), w = fits(ceil8(N), K);
+  if (x && w && ragged_pays(M, K)) r.products |= products & kFwd;
+  if (dy && w && ragged_pays(M, N)) r.products |= products & kDgrad;
+  if (x && dy) r.products |= products & kWgrad;
+  if (K % 8 != 0 && (r.products & (kFwd | kWgrad))) r.x = round256((size_t)M * ceil8(K) * 2);
+  if (N % 8 != 0 && (r.products & (kDgrad | kWgrad))) r.dy = round256((size_t)M * ceil8(N) * 2);
+  if (r.products & (kFwd | kDgrad)) r.w = round256((size_t)ceil8(N) * ceil8(K) * 2);
   r.total = r.x + r.dy + r.w;
   return r;
 }
@@ -515,71 +524,83 @@ static void pad_rows_launch(bool packed, const void* src, int64_t ld, int64_t ro
                        nullptr, 0, dst, drows, dcols);
 }
 
-// The padded operands of one call, made on first use at the workspace's end
-// (`inner` bytes before them stay for the products' split-K partials).
+// The padded operands of one call, at the workspace's end (`inner` bytes before
+// them stay for the products' split-K partials).
 struct Ragged {
   char* base = nullptr;
   size_t inner = 0;
-  RaggedRoom room{0, 0, 0, 0};
+  RaggedRoom room{0, 0, 0, 0, 0};
   hipStream_t st;
-  // false: the shape is not ragged, or the workspace has no room
-  bool init(int64_t M, int64_t N, int64_t K, void* workspace, size_t ws_bytes, hipStream_t stream) {
-    room = ragged_room(M, N, K);
+  // false: none of the products runs on copies, or the workspace has no room
+  bool init(int64_t M, int64_t N, int64_t K, int products, void* workspace, size_t ws_bytes, hipStream_t stream) {
+    room = ragged_room(M, N, K, products);
     st = stream;
-    if (room.total == 0 || !workspace || ws_bytes < kSplitkCounterBytes + room.total + 256) return false;
+    if (room.products == 0 || !workspace || ws_bytes < kSplitkCounterBytes + room.total + 256) return false;
     inner = (ws_bytes - room.total) / 256 * 256;
     base = (char*)workspace + inner;
     return true;
   }
-  static bool plain(const uint16_t* p, int64_t ld, int64_t cols) {
-    return cols % 8 == 0 && ld % 8 == 0 && ((uintptr_t)p % 16) == 0;
-  }
-  // (p, ld) of an activation operand, replaced by a padded copy where needed
-  void activation(const uint16_t*& p, int64_t& ld, int64_t rows, int64_t cols, size_t off) const {
-    if (plain(p, ld, cols)) return;
-    uint16_t* d = (uint16_t*)(base + off);
-    pad_rows_launch(false, p, ld, rows, cols, nullptr, nullptr, 0, d, rows, st);
-    p = d;
+  // (p, ld), an activation operand of cols columns, becomes its copy's place
+  // where it needs a copy (`copy` set); false where that has no room (an operand
+  // of whole chunks whose base or pitch the fast kernels cannot read)
+  static bool place(const uint16_t*& p, int64_t& ld, int64_t cols, char* at, size_t bytes, bool& copy) {
+    copy = !(cols % 8 == 0 && ld % 8 == 0 && ((uintptr_t)p % 16) == 0);
+    if (!copy) return true;
+    p = (const uint16_t*)at;
     ld = ceil8(cols);
+    return bytes != 0;
   }
-  void x(const uint16_t*& p, int64_t& ld, int64_t M, int64_t K) const { activation(p, ld, M, K, 0); }
-  void dy(const uint16_t*& p, int64_t& ld, int64_t M, int64_t N) const { activation(p, ld, M, N, room.x); }
-  // the weight operand of g (packed words, or bf16 rows) as padded bf16 rows
-  const uint16_t* weight(const GemmArgs& g, bool packed, int64_t N, int64_t K) const {
-    uint16_t* d = (uint16_t*)(base + room.x + room.dy);
-    pad_rows_launch(packed, g.b, g.ldb, N, K, g.row_exp, g.col_exp, g.bias, d, ceil8(N), st);
-    return d;
+  bool x(const uint16_t*& p, int64_t& ld, int64_t K, bool& copy) const { return place(p, ld, K, base, room.x, copy); }
+  bool dy(const uint16_t*& p, int64_t& ld, int64_t N, bool& copy) const {
+    return place(p, ld, N, base + room.x, room.dy, copy);
+  }
+  uint16_t* w() const { return (uint16_t*)(base + room.x + room.dy); }
+  void copy(const uint16_t* src, int64_t ld, int64_t rows, int64_t cols, const uint16_t* dst) const {
+    pad_rows_launch(false, src, ld, rows, cols, nullptr, nullptr, 0, (uint16_t*)dst, rows, st);
   }
 };
 
 static bool ragged_out(const GemmArgs& g) { return g.ldc % 4 != 0 || g.J % 4 != 0 || ((uintptr_t)g.c % 8) != 0; }
 
-// forward or dgrad of a ragged layer on its padded operands; -1 where the
-// fast kernels do not take them either
+// forward or dgrad of a ragged layer on its padded operands; -1, with nothing
+// copied, where it does not run on them
 template <int MODE>
 static int ragged_product(const Ragged& rg, const GemmArgs& g, void* workspace, const char* what) {
-  constexpr bool FWD = MODE == MODE_FWD || MODE == MODE_FWD_BF16;
+  constexpr bool FWD = MODE == MODE_FWD || MODE == MODE_FWD_BF16, PACKED = MODE == MODE_FWD || MODE == MODE_DGRAD;
+  if (!(rg.room.products & (FWD ? kFwd : kDgrad))) return -1;
   GemmArgs p = g;
   const int64_t M = g.I, N = FWD ? g.J : g.R, K = FWD ? g.R : g.J;
-  if (FWD) rg.x(p.a, p.lda, M, K);
-  else rg.dy(p.a, p.lda, M, N);
-  p.b = rg.weight(g, MODE == MODE_FWD || MODE == MODE_DGRAD, N, K);
+  bool copy;
+  if (!(FWD ? rg.x(p.a, p.lda, K, copy) : rg.dy(p.a, p.lda, N, copy))) return -1;
+  p.b = rg.w();
   p.ldb = ceil8(K);
   p.R = ceil8(g.R);
   p.row_exp = p.col_exp = nullptr;
   p.pad = 1;
   p.sc = ragged_out(g);
-  return gemm_fast_launch(FWD ? MODE_FWD_BF16 : MODE_DGRAD_BF16, p, workspace, rg.inner, rg.st, what);
+  constexpr int mode = FWD ? MODE_FWD_BF16 : MODE_DGRAD_BF16;
+  if (!gemm_fast_takes(mode, p)) return -1;
+  if (copy) rg.copy(g.a, g.lda, M, g.R, p.a);
+  pad_rows_launch(PACKED, g.b, g.ldb, N, K, g.row_exp, g.col_exp, g.bias, rg.w(), ceil8(N), rg.st);
+  return gemm_fast_launch(mode, p, workspace, rg.inner, rg.st, what);
 }
 
-// g (a WGRAD) on padded dy and x
-static void ragged_wgrad(const Ragged& rg, GemmArgs& g) {
+// g (a WGRAD) on padded dy and x; false, with nothing copied, where it does not
+// run on them
+static bool ragged_wgrad(const Ragged& rg, GemmArgs& g) {
+  if (!(rg.room.products & kWgrad)) return false;
+  GemmArgs p = g;
   const uint16_t* x = (const uint16_t*)g.b;
-  rg.dy(g.a, g.lda, g.R, g.I);
-  rg.x(x, g.ldb, g.R, g.J);
-  g.b = x;
-  g.pad = 1;
-  g.sc = ragged_out(g);
+  bool copy_dy, copy_x;
+  if (!rg.dy(p.a, p.lda, g.I, copy_dy) || !rg.x(x, p.ldb, g.J, copy_x)) return false;
+  p.b = x;
+  p.pad = 1;
+  p.sc = ragged_out(g);
+  if (!gemm_fast_takes(MODE_WGRAD, p)) return false;
+  if (copy_dy) rg.copy(g.a, g.lda, g.R, g.I, p.a);
+  if (copy_x) rg.copy((const uint16_t*)g.b, g.ldb, g.R, g.J, x);
+  g = p;
+  return true;
 }
 
 // room of a layer's decoded weight (0: neither product decodes)
@@ -612,7 +633,7 @@ static bool decoded(int mode, const GemmArgs& g, void* workspace, size_t ws_byte
 // workspace: their caller gives each call a workspace of its own, and need not
 // clear it.
 static bool own_workspace(int64_t M, int64_t N, int64_t K, bool packed) {
-  return ragged_room(M, N, K).total != 0 || (packed && decode_room(M, N, K) != 0);
+  return ragged_room(M, N, K).products != 0 || (packed && decode_room(M, N, K) != 0);
 }
 
 __global__ __launch_bounds__(256) void clear_counters_kernel(uint32_t* c, int n) {
@@ -628,13 +649,12 @@ static int launch_gemm(GemmArgs g, void* workspace, size_t ws_bytes, hipStream_t
     constexpr bool FWD = MODE == MODE_FWD || MODE == MODE_FWD_BF16;
     Ragged rg;
     if (MODE == MODE_WGRAD) {
-      if (rg.init(g.R, g.I, g.J, workspace, ws_bytes, st)) {
-        GemmArgs p = g;
-        ragged_wgrad(rg, p);
+      GemmArgs p = g;
+      if (rg.init(g.R, g.I, g.J, kWgrad, workspace, ws_bytes, st) && ragged_wgrad(rg, p)) {
         const int rc = gemm_fast_launch(MODE, p, workspace, rg.inner, st, what);
         if (rc != -1) return rc;
       }
-    } else if (!g.ay && ragged_pays(g.I, g.R) && rg.init(g.I, FWD ? g.J : g.R, FWD ? g.R : g.J, workspace, ws_bytes, st)) {
+    } else if (!g.ay && rg.init(g.I, FWD ? g.J : g.R, FWD ? g.R : g.J, FWD ? kFwd : kDgrad, workspace, ws_bytes, st)) {
       const int rc = ragged_product<MODE>(rg, g, workspace, what);
       if (rc != -1) return rc;
     }
@@ -744,11 +764,13 @@ size_t gemm_splitk_need(int mode, int64_t I, int64_t J, int64_t R) {
 }
 
 size_t gemm_bf16_need(int mode, int64_t I, int64_t J, int64_t R) {
-  const bool fwd = mode == MODE_FWD_BF16;
   const size_t plain = gemm_splitk_need(mode, I, J, R);
-  const RaggedRoom r = fwd ? ragged_room(I, J, R) : ragged_room(I, R, J);
-  if (r.total == 0) return plain;
-  const size_t part = gemm_fast_partial_bytes(mode, I, J, R, plan_gemm(I, J, R, true).splits);
+  const RaggedRoom r = mode == MODE_WGRAD      ? ragged_room(R, I, J, kWgrad)
+                       : mode == MODE_FWD_BF16 ? ragged_room(I, J, R, kFwd)
+                                               : ragged_room(I, R, J, kDgrad);
+  if (r.products == 0) return plain;
+  const int keep = mode == MODE_WGRAD ? 0 : plan_gemm(I, J, R, true).splits;
+  const size_t part = gemm_fast_partial_bytes(mode, I, J, R, keep);
   return std::max(plain, kSplitkCounterBytes + round256(part) + r.total + 256);
 }
 
@@ -767,7 +789,7 @@ extern "C" size_t concord_gemm_workspace_need(int64_t M, int64_t N, int64_t K, i
                    splitk_partials(MODE_DGRAD, M, K, N), splitk_partials(MODE_DGRAD_BF16, M, K, N)})
     if (v > m) m = v;
   const RaggedRoom r = ragged_room(M, N, K);
-  if (r.total) {   // the padded operands, and the partials of the products on them
+  if (r.products) {   // the padded operands, and the partials of the products on them
     const int64_t N8 = ceil8(N), K8 = ceil8(K);
     for (size_t v : {splitk_partials(MODE_FWD_BF16, M, N, K8), splitk_partials(MODE_DGRAD_BF16, M, K, N8)})
       if (v > m) m = v;
@@ -860,17 +882,12 @@ static int wgrad_vhat_impl(const GemmArgs* gd, const uint16_t* dy, int64_t ld_dy
   GemmArgs pend;        // a dgrad split-K reduction the finalize launch carries
   int pend_rbi = 0;
   Ragged rg;
-  GemmArgs gdr;
-  if (!gemm_fast_takes(MODE_WGRAD, g) && rg.init(M, N, K, gemm_workspace, gemm_workspace_bytes, st)) {
-    // dy and x padded once, for both products
-    ragged_wgrad(rg, g);
+  if (!gemm_fast_takes(MODE_WGRAD, g) &&
+      rg.init(M, N, K, gd ? kDgrad | kWgrad : kWgrad, gemm_workspace, gemm_workspace_bytes, st) &&
+      ragged_wgrad(rg, g)) {
     if (gd && gd->I > 0 && gd->J > 0) {
-      gdr = *gd;
-      gdr.a = g.a;
-      gdr.lda = g.lda;
-      if (!gemm_fast_takes(MODE_DGRAD, gdr) && ragged_pays(gd->I, gd->R))
-        rc = ragged_product<MODE_DGRAD>(rg, gdr, gemm_workspace, what);
-      if (rc == -1) rc = launch_gemm<MODE_DGRAD>(gdr, gemm_workspace, rg.inner, st, what);
+      if (!gemm_fast_takes(MODE_DGRAD, *gd)) rc = ragged_product<MODE_DGRAD>(rg, *gd, gemm_workspace, what);
+      if (rc == -1) rc = launch_gemm<MODE_DGRAD>(*gd, gemm_workspace, rg.inner, st, what);
       if (rc != CONCORD_OK) return rc;
       rc = -1;
     }

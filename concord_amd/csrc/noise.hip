@@ -245,7 +245,7 @@ static SigmagLayout sigmag_layout(int64_t M, int64_t N, int64_t K) {
   size_t o = 0;
   // the product's split-K region first: its tile counters sit at the
   // workspace's start for every shape (see muon_layout)
-  L.gemm = o; o += r256(gemm_splitk_need(MODE_WGRAD, N, K, M));
+  L.gemm = o; o += r256(gemm_bf16_need(MODE_WGRAD, N, K, M));
   L.dyt = o; o += r256((size_t)M * N * 2);
   L.prod = o; o += r256((size_t)N * K * 2);
   L.part = o; o += r256((size_t)2 * cdiv(N * K, kNoiseBlock) * 4);

@@ -165,3 +165,24 @@ def test_split_counters_of_an_uncleared_workspace(M, N, K):
     assert torch.equal(*outs)
     ref = dy.double().T @ x.double()
     assert ((outs[0].double() - ref).norm() / ref.norm()).item() < 2.0 ** -8
+
+
+def test_ragged_operand_beyond_the_extents():
+    """dy's padded copy would pass the 2^30 bytes that the fast kernels address:
+    the dgrad and the weight gradient run on the operands as they are."""
+    from concord_amd import packed_b as pb
+    M, N, K = 1 << 20, 513, 9
+    gen = torch.Generator(device=DEV).manual_seed(0)
+    x = torch.randn(M, K, device=DEV, generator=gen).to(torch.bfloat16)
+    dy = torch.randn(M, N, device=DEV, generator=gen).to(torch.bfloat16)
+    W = torch.randn(N, K, device=DEV, generator=gen).to(torch.bfloat16)
+    y = pb._gemm_fwd(x, None, None, None, 15, None, W)
+    dx = pb._gemm_dgrad(dy, None, None, None, 15, W)
+    gw = pb._wgrad(dy, x)
+    sync()
+    for at in (slice(0, 1000), slice(M - 1000, M)):
+        for got, a, b in ((y[at], x[at], W.T), (dx[at], dy[at], W)):
+            ref, terms = a.double() @ b.double(), a.double().abs() @ b.double().abs()
+            assert ((got.double() - ref).abs() <= ref.abs() * 2.0 ** -8 + terms * a.shape[1] * 2.0 ** -24).all()
+    ref = sum(dy[i:i + 65536].double().T @ x[i:i + 65536].double() for i in range(0, M, 65536))
+    assert ((gw.double() - ref).norm() / ref.norm()).item() < 2.0 ** -8

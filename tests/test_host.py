@@ -234,3 +234,21 @@ def test_calls_that_write_operands_get_a_workspace_of_their_own(L):
     for M, N, K in [(308, 1280, 2048), (3, 5, 7)]:
         assert pb._gemm_workspace("cpu", M, N, K) is pb._gemm_workspace("cpu", M, N, K)
     pb._GEMM_WORKSPACES.pop("cpu")
+
+
+@pytest.mark.parametrize("M,N,K,copied", [
+    (16384, 50257, 768, 50264 * 768 * 2),            # dy's copy would pass 2^30 bytes: the weight's alone, for the forward
+    (16384, 768, 50257, 768 * 50264 * 2),            # x's likewise: the weight's, for the dgrad
+    (16384, 65, 384, 16384 * 72 * 2 + 72 * 384 * 2),   # x has whole chunks
+    (2048, 320, 36, 2048 * 40 * 2 + 320 * 40 * 2),     # dy has
+    (4, 33, 31, 4 * 32 * 2 + 4 * 40 * 2),              # too few rows and terms for the forward and the dgrad
+])
+def test_workspace_holds_the_copies_that_are_made(L, M, N, K, copied):
+    """The room of a ragged layer's padded copies: none for an operand that is
+    used as it is, nor for one that the fast kernels could not address."""
+    N8, K8 = -(-N // 8) * 8, -(-K // 8) * 8
+    # the split-K partials of the layer and of its padded twin bound the rest
+    rest = max(L.concord_gemm_workspace_need(M, n, k, 0, None) for n in (N8, N8 - 4, N) for k in (K8, K8 - 4, K)
+               if n % 8 == 0 and k % 8 == 0)
+    need = L.concord_gemm_workspace_bytes(M, N, K)
+    assert copied <= need <= copied + rest + 4 * 256
