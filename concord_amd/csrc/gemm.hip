@@ -541,10 +541,12 @@ struct Ragged {
     return true;
   }
   // (p, ld), an activation operand of cols columns, becomes its copy's place
-  // where it needs a copy (`copy` set); false where that has no room (an operand
-  // of whole chunks whose base or pitch the fast kernels cannot read)
+  // where it needs a copy (`copy` set, unless p is that copy, made for the
+  // product before); false where that has no room (an operand of whole chunks
+  // whose base or pitch the fast kernels cannot read)
   static bool place(const uint16_t*& p, int64_t& ld, int64_t cols, char* at, size_t bytes, bool& copy) {
-    copy = !(cols % 8 == 0 && ld % 8 == 0 && ((uintptr_t)p % 16) == 0);
+    const bool made = bytes != 0 && p == (const uint16_t*)at;
+    copy = !made && !(cols % 8 == 0 && ld % 8 == 0 && ((uintptr_t)p % 16) == 0);
     if (!copy) return true;
     p = (const uint16_t*)at;
     ld = ceil8(cols);
@@ -886,7 +888,10 @@ static int wgrad_vhat_impl(const GemmArgs* gd, const uint16_t* dy, int64_t ld_dy
       rg.init(M, N, K, gd ? kDgrad | kWgrad : kWgrad, gemm_workspace, gemm_workspace_bytes, st) &&
       ragged_wgrad(rg, g)) {
     if (gd && gd->I > 0 && gd->J > 0) {
-      if (!gemm_fast_takes(MODE_DGRAD, *gd)) rc = ragged_product<MODE_DGRAD>(rg, *gd, gemm_workspace, what);
+      GemmArgs gdr = *gd;   // (dy padded once, for both products)
+      gdr.a = g.a;
+      gdr.lda = g.lda;
+      if (!gemm_fast_takes(MODE_DGRAD, *gd)) rc = ragged_product<MODE_DGRAD>(rg, gdr, gemm_workspace, what);
       if (rc == -1) rc = launch_gemm<MODE_DGRAD>(*gd, gemm_workspace, rg.inner, st, what);
       if (rc != CONCORD_OK) return rc;
       rc = -1;

@@ -186,3 +186,23 @@ def test_ragged_operand_beyond_the_extents():
             assert ((got.double() - ref).abs() <= ref.abs() * 2.0 ** -8 + terms * a.shape[1] * 2.0 ** -24).all()
     ref = sum(dy[i:i + 65536].double().T @ x[i:i + 65536].double() for i in range(0, M, 65536))
     assert ((gw.double() - ref).norm() / ref.norm()).item() < 2.0 ** -8
+
+
+@pytest.mark.parametrize("M,N,K,copies", [(512, 65, 384, 2), (600, 65, 37, 3), (640, 320, 36, 1)])
+def test_backward_pads_each_operand_once(M, N, K, copies):
+    """Copies a ragged backward launches: dy and x where their widths are no
+    whole chunks, and the weight where the dgrad reads it padded."""
+    from torch.profiler import ProfilerActivity, profile
+    from concord_amd import packed_b as pb
+    rng = np.random.default_rng(N)
+    pk, red, ced = (dev(t) for t in rand_state(rng, N, K, exp=(-2, 2), col=(-1, 1)))
+    x = torch.randn(M, K, device=DEV).to(torch.bfloat16)
+    dy = torch.randn(M, N, device=DEV).to(torch.bfloat16)
+    args = (torch.ones(N, device=DEV), torch.ones(K, device=DEV), torch.ones(1, device=DEV), 0.999, None, None,
+            torch.ones(1, dtype=torch.int32, device=DEV))
+    pb._dgrad_wgrad_vhat(dy, x, pk, red, ced, 15, *args, with_bias=True)
+    sync()
+    with profile(activities=[ProfilerActivity.CUDA]) as prof:
+        pb._dgrad_wgrad_vhat(dy, x, pk, red, ced, 15, *args, with_bias=True)
+        sync()
+    assert sum(e.count for e in prof.key_averages() if "pad_rows_kernel" in e.key) == copies
