@@ -237,9 +237,9 @@ _GEMM_WORKSPACES = {}
 # the sizes below are functions of the problem alone; a call plans every product
 # of the layer (5 - 20 us), so they are kept per problem
 @functools.lru_cache(maxsize=4096)
-def _gemm_need(M, N, K):
+def _gemm_need(M, N, K, packed):
     own = ctypes.c_int(0)
-    need = C.lib().concord_gemm_workspace_need(M, N, K, 1, ctypes.byref(own))
+    need = C.lib().concord_gemm_workspace_need(M, N, K, packed, ctypes.byref(own))
     return int(need), bool(own.value)
 
 
@@ -248,14 +248,16 @@ def _need(N, K, M):
     return int(C.lib().concord_workspace_bytes(N, K, M))
 
 
-def _gemm_workspace(device, M, N, K):
+def _gemm_workspace(device, M, N, K, packed=True):
     """Zero-initialised per-device split-K workspace of the GEMMs, grown to the
     largest problem seen (grow it eagerly, before any graph capture).  A call
     that writes operands into its workspace (padded copies of a ragged layer's,
     a decoded weight) gets one of its own from the allocator: forwards on
-    several streams, or in a graph beside eager ones, must not share it."""
+    several streams, or in a graph beside eager ones, must not share it.
+    packed: a forward or dgrad of packed words is among the call's products
+    (not a cached bf16 weight, nor the weight gradient alone)."""
     key = _dev_key(device)
-    need, own = _gemm_need(int(M), int(N), int(K))
+    need, own = _gemm_need(int(M), int(N), int(K), packed)
     if own:
         return torch.empty(need, dtype=torch.uint8, device=key)
     ws = _GEMM_WORKSPACES.get(key)
@@ -518,7 +520,7 @@ def _gemm_fwd(x2, packed_w, row_exp, col_exp, mantissa_bias, bias, weight_buf):
     N = (weight_buf if weight_buf is not None else packed_w).shape[0]
     y = torch.empty((M, N), dtype=torch.bfloat16, device=x2.device)
     st = C.stream_of(x2.device)
-    ws = _gemm_workspace(x2.device, M, N, K)
+    ws = _gemm_workspace(x2.device, M, N, K, weight_buf is None)
     if weight_buf is None:
         C.check(C.lib().concord_dqgemm_fwd(
             C.ptr(x2), x2.stride(0), C.ptr(packed_w), packed_w.stride(0), C.ptr(row_exp),
@@ -536,7 +538,7 @@ def _gemm_dgrad(dy, packed_w, row_exp, col_exp, mantissa_bias, weight_buf):
     K = (weight_buf if weight_buf is not None else packed_w).shape[1]
     dx = torch.empty((M, K), dtype=torch.bfloat16, device=dy.device)
     st = C.stream_of(dy.device)
-    ws = _gemm_workspace(dy.device, M, N, K)
+    ws = _gemm_workspace(dy.device, M, N, K, weight_buf is None)
     if weight_buf is None:
         C.check(C.lib().concord_dqgemm_dgrad(
             C.ptr(dy), dy.stride(0), C.ptr(packed_w), packed_w.stride(0), C.ptr(row_exp),
@@ -553,7 +555,7 @@ def _wgrad(dy, x2):
     M, N = dy.shape
     K = x2.shape[1]
     gw = torch.empty((N, K), dtype=torch.bfloat16, device=dy.device)
-    ws = _gemm_workspace(dy.device, M, N, K)
+    ws = _gemm_workspace(dy.device, M, N, K, False)
     C.check(C.lib().concord_wgrad(C.ptr(dy), dy.stride(0), C.ptr(x2), x2.stride(0), C.ptr(gw),
                                   gw.stride(0), M, N, K, C.ptr(ws), ws.numel(),
                                   C.stream_of(dy.device)), "wgrad")
@@ -570,7 +572,7 @@ def _wgrad_vhat(dy, x2, v_row, v_col, sum_v_inv, beta2, row_max, col_max, salt_c
     K = x2.shape[1]
     gw = torch.empty((N, K), dtype=torch.bfloat16, device=dy.device)
     gb = torch.empty(N, dtype=torch.bfloat16, device=dy.device) if with_bias else None
-    gws = _gemm_workspace(dy.device, M, N, K)
+    gws = _gemm_workspace(dy.device, M, N, K, False)
     ws = _workspace(dy.device, N, K, M if with_bias else 0)
     C.check(C.lib().concord_wgrad_vhat(
         C.ptr(dy), dy.stride(0), C.ptr(x2), x2.stride(0), C.ptr(gw), gw.stride(0), M, N, K,
@@ -590,7 +592,7 @@ def _dgrad_wgrad_vhat(dy, x2, packed_w, row_exp, col_exp, mantissa_bias, v_row, 
     dx = torch.empty((M, K), dtype=torch.bfloat16, device=dy.device)
     gw = torch.empty((N, K), dtype=torch.bfloat16, device=dy.device)
     gb = torch.empty(N, dtype=torch.bfloat16, device=dy.device) if with_bias else None
-    gws = _gemm_workspace(dy.device, M, N, K)
+    gws = _gemm_workspace(dy.device, M, N, K, True)
     ws = _workspace(dy.device, N, K, M if with_bias else 0)
     C.check(C.lib().concord_dgrad_wgrad_vhat(
         C.ptr(dy), dy.stride(0), C.ptr(packed_w), packed_w.stride(0), C.ptr(row_exp), C.ptr(col_exp),
@@ -617,7 +619,7 @@ def _dgrad_wgrad_update(ctx, dy, x2, fuse=False):
     dx = torch.empty((M, K), dtype=torch.bfloat16, device=dev)
     gw = torch.empty((N, K), dtype=torch.bfloat16, device=dev)
     gb = torch.empty(N, dtype=torch.bfloat16, device=dev) if ctx.has_bias else None
-    gws = _gemm_workspace(dev, M, N, K)
+    gws = _gemm_workspace(dev, M, N, K, True)
     ws = _workspace(dev, N, K, M if ctx.has_bias else 0)
     dcc = ctx.drift_cancel_C
     if dcc is None:

@@ -227,12 +227,18 @@ def test_calls_that_write_operands_get_a_workspace_of_their_own(L):
     calls) must not hold the same buffer."""
     from concord_amd import packed_b as pb
     for M, N, K in [(2048, 320, 36), (512, 65, 384), (4096, 1280, 1280)]:
-        a, b = (pb._gemm_workspace("cpu", M, N, K) for _ in range(2))
+        a, b = (pb._gemm_workspace("cpu", M, N, K, True) for _ in range(2))
         assert a.numel() == b.numel() >= L.concord_gemm_workspace_bytes(M, N, K)
         assert a.data_ptr() != b.data_ptr(), (M, N, K)
+    # a cached bf16 weight and the weight gradient alone decode nothing: no room
+    # for a decoded weight, and the device's buffer
+    cached = pb._gemm_workspace("cpu", 4096, 1280, 1280, False)
+    assert cached is pb._gemm_workspace("cpu", 4096, 1280, 1280, False)
+    assert (L.concord_gemm_workspace_need(4096, 1280, 1280, 0, None) + 1280 * 1280 * 2
+            <= L.concord_gemm_workspace_need(4096, 1280, 1280, 1, None))
     # nothing is copied: the zeroed buffer of the device, its tile counters in use
     for M, N, K in [(308, 1280, 2048), (3, 5, 7)]:
-        assert pb._gemm_workspace("cpu", M, N, K) is pb._gemm_workspace("cpu", M, N, K)
+        assert pb._gemm_workspace("cpu", M, N, K, True) is pb._gemm_workspace("cpu", M, N, K, True)
     pb._GEMM_WORKSPACES.pop("cpu")
 
 
