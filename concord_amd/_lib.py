@@ -167,9 +167,12 @@ def ptr(t):
 
 def stream_of(device):
     """Handle of the device's current stream (the raw handle: building the
-    Stream object around it took 4 us of a launch's host time)."""
-    index = device.index if isinstance(device, torch.device) else torch.device(device).index
-    return torch._C._cuda_getCurrentRawStream(torch.cuda.current_device() if index is None else index)
+    Stream object around it took 4 us of a launch's host time).  Raises for
+    any other device: its tensors' addresses must not reach a kernel."""
+    d = device if isinstance(device, torch.device) else torch.device(device)
+    if d.type != "cuda":
+        raise ValueError(f"Expected a cuda device, but got: {d}")
+    return torch._C._cuda_getCurrentRawStream(torch.cuda.current_device() if d.index is None else d.index)
 
 
 def require_device_tensor(t, name):

@@ -112,6 +112,22 @@ def test_wrappers_refuse_cpu_tensors():
                                    torch.empty(4, 8, dtype=torch.bfloat16))
 
 
+@pytest.mark.parametrize("device", ["cpu", "meta"])
+def test_products_refuse_tensors_of_other_devices(device):
+    """No host address may reach a launch: the stream lookup of every product
+    refuses the device, as torch.cuda.current_stream does."""
+    from concord_amd import _lib as C, packed_b as pb
+    x, dy = (torch.empty(16, k, dtype=torch.bfloat16, device=device) for k in (24, 8))
+    W = torch.empty(8, 24, dtype=torch.bfloat16, device=device)
+    packed = (torch.empty(8, 24, dtype=torch.int32, device=device), torch.empty(8, dtype=torch.int8, device=device),
+              torch.empty(24, dtype=torch.int8, device=device), 15)
+    for call in (lambda: C.stream_of(torch.device(device)), lambda: C.stream_of(device),
+                 lambda: pb._gemm_fwd(x, *packed, None, None), lambda: pb._gemm_dgrad(dy, *packed, W),
+                 lambda: pb._wgrad(dy, x), lambda: pb._bias_grad(dy)):
+        with pytest.raises(ValueError, match="Expected a cuda device"):
+            call()
+
+
 def test_public_api_surface():
     """Names a user of concord/__init__.py:7-31 imports exist with the same meaning."""
     import concord_amd as ca
