@@ -2418,11 +2418,14 @@ size_t gemm_fast_partial_bytes(int mode, int64_t I, int64_t J, int64_t R, int ke
 // dgrad, packed kernel -> decode + bf16 kernel, us: 4096 x 1280 x 10240 138 ->
 // 109, 16384 x 640 x 640 29.5 -> 23.8, 8192 x 640 x 5120 71.7 -> 56.8,
 // 2048 x 5120 x 1280 45.2 -> 39.0 (training steps of those layers 2 - 6%
-// shorter).  Forward: 8192 x 5120 x 640 82.6 -> 67.6, but training steps whose
-// forward also decoded were 1 - 3% longer at 4096 x 1280 x 1280,
-// 4096 x 10240 x 1280 and 16384 x 640 x 640, where the pass reads a weight no
-// cache holds and the chip's clock, not the producers, sets the product's pace.
-// Below 4e9 products the pass's fixed time takes the gain.  A split dgrad
+// shorter).  Forward (rows x N x K), alone and in a training step, without ->
+// with the decode: 16384 x 1280 x 1280 67.5 -> 59.2 and 249 -> 239, 16384 x 2560
+// x 640 85.2 -> 67.0 and 261 -> 253, 12288 x 2560 x 1280 99.9 -> 78.1 and 336 ->
+// 309, 8192 x 5120 x 640 84.1 -> 68.8 and 270 -> 265, 8192 x 640 x 5120 75.8 ->
+// 69.3 and 282 -> 278, 8192 x 1280 x 5120 114 -> 102 and 417 -> 408; two steps
+// lose, 8192 x 2560 x 1280 (67.5 -> 60.4 but 255 -> 260) and 8192 x 5120 x 1280
+// (134 -> 119 but 428 -> 437).  Below the rule's line the steps lose by 1 - 3%:
+// 4096 x 1280 x 1280, 4096 x 10240 x 1280, 16384 x 640 x 640.  Below 4e9 products the pass's fixed time takes the gain.  A split dgrad
 // keeps the packed kernel: the WGRAD launch carries its reduction
 // (2048 x 1280 x 5120: 42.8 -> 42 without that).
 bool gemm_decode_pays(int mode, int64_t I, int64_t J, int64_t R) {

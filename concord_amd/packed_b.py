@@ -256,10 +256,10 @@ def _gemm_workspace(device, M, N, K, packed=True):
     several streams, or in a graph beside eager ones, must not share it.
     packed: a forward or dgrad of packed words is among the call's products
     (not a cached bf16 weight, nor the weight gradient alone)."""
-    key = _dev_key(device)
     need, own = _gemm_need(int(M), int(N), int(K), packed)
     if own:
-        return torch.empty(need, dtype=torch.uint8, device=key)
+        return torch.empty(need, dtype=torch.uint8, device=device)
+    key = _dev_key(device)
     ws = _GEMM_WORKSPACES.get(key)
     if ws is None or ws.numel() < need:
         ws = torch.zeros(need, dtype=torch.uint8, device=key)
