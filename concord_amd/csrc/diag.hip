@@ -35,9 +35,10 @@ __device__ __forceinline__ i32x4 rsrc(const void* p, uint32_t bytes) {
   for (int e = 0; e < 4; ++e) r[e] = __builtin_amdgcn_readfirstlane(r[e]);
   return r;
 }
-// lane l's 16 bytes at voff land at LDS lds_base + 16 l
+// lane l's 16 bytes at voff land at LDS lds_base + 16 l (the s_nop: M0 needs a
+// wait state between its write and the load that reads it)
 __device__ __forceinline__ void dma16(i32x4 rs, uint32_t voff, uint32_t lds_base) {
-  asm volatile("s_mov_b32 m0, %2\n\tbuffer_load_dwordx4 %0, %1, 0 offen lds"
+  asm volatile("s_mov_b32 m0, %2\n\ts_nop 0\n\tbuffer_load_dwordx4 %0, %1, 0 offen lds"
                :
                : "v"(voff), "s"(rs), "s"(lds_base)
                : "memory", "m0");

@@ -45,10 +45,10 @@ struct FarBase {
   CONCORD_DEV const lds_char* at(uint32_t o) const { return lds_at(o >= 65536u ? hi : lo) + (o & 65535u); }
 };
 
-// dma16 to LDS address base + OFF
+// dma16 to LDS address base + OFF (the s_nop: M0's wait state, as there)
 template <int OFF>
 CONCORD_DEV void dma16_at(i32x4 rsrc, uint32_t voff, uint32_t soff, uint32_t base) {
-  asm volatile("s_add_u32 m0, %3, %4\n\tbuffer_load_dwordx4 %0, %1, %2 offen lds"
+  asm volatile("s_add_u32 m0, %3, %4\n\ts_nop 0\n\tbuffer_load_dwordx4 %0, %1, %2 offen lds"
                :
                : "v"(voff), "s"(rsrc), "s"(soff), "s"(base), "n"(OFF)
                : "memory", "m0", "scc");

@@ -1083,9 +1083,11 @@ typedef __attribute__((address_space(3))) void* lds_ptr_t;
 // One LDS-DMA buffer load, issued as inline assembly so the compiler does not
 // track it: it cannot tell which ring slot a DMA writes and would otherwise
 // wait for every outstanding DMA before any LDS read.  The kernel waits for
-// its DMAs itself (vmcnt) before each barrier and before it ends.
+// its DMAs itself (vmcnt) before each barrier and before it ends.  The hardware
+// needs a wait state between a scalar write of M0 and an LDS-DMA that reads it
+// (the compiler puts one there for its own; it adds none inside inline asm).
 CONCORD_DEV void dma16(i32x4 rsrc, uint32_t voff, uint32_t soff, uint32_t lds_base) {
-  asm volatile("s_mov_b32 m0, %3\n\tbuffer_load_dwordx4 %0, %1, %2 offen lds"
+  asm volatile("s_mov_b32 m0, %3\n\ts_nop 0\n\tbuffer_load_dwordx4 %0, %1, %2 offen lds"
                :
                : "v"(voff), "s"(rsrc), "s"(soff), "s"(lds_base)
                : "memory", "m0");

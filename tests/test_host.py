@@ -274,3 +274,21 @@ def test_workspace_holds_the_copies_that_are_made(L, M, N, K, copied):
                if n % 8 == 0 and k % 8 == 0)
     need = L.concord_gemm_workspace_bytes(M, N, K)
     assert copied <= need <= copied + rest + 4 * 256
+
+
+def test_lds_dma_waits_for_m0():
+    """An LDS-DMA reads its LDS address from M0 and needs a wait state after the
+    scalar write of it; the compiler adds none inside inline asm."""
+    import glob
+    csrc = os.path.join(os.path.dirname(os.path.dirname(os.path.abspath(__file__))), "concord_amd", "csrc")
+    found = 0
+    for path in glob.glob(os.path.join(csrc, "*")):
+        for text in re.findall(r'asm volatile\("([^"]*)"', open(path).read()):
+            lines = [l.strip() for l in text.replace("\\t", "").split("\\n")]
+            for i, l in enumerate(lines):
+                if re.search(r"\blds$", l):
+                    found += 1
+                    before = lines[:i]
+                    assert before and before[-1].startswith("s_nop"), (os.path.basename(path), lines)
+                    assert re.match(r"s_\w+ m0,", before[-2]), (os.path.basename(path), lines)
+    assert found >= 3
