@@ -471,8 +471,11 @@ struct RaggedRoom { int products; size_t x, dy, w, total; };
 static RaggedRoom ragged_room(int64_t M, int64_t N, int64_t K, int products = kFwd | kDgrad | kWgrad) {
   RaggedRoom r{0, 0, 0, 0, 0};
   if ((double)M * (double)N * (double)K < kRaggedWork || (N % 8 == 0 && K % 8 == 0)) return r;
-  auto fits = [](int64_t rows, int64_t cols) { return rows < (1LL << 29) / ceil8(cols); };
-  const bool x = fits(M, K), dy = fits(M, N), w = fits(ceil8(N), K);
+  // ((rows - 1) * ceil8(cols) + cols) * 2 < 2^30
+  auto fits = [](int64_t rows, int64_t cols) {
+    return cols < (1LL << 29) && rows - 1 <= ((1LL << 29) - 1 - cols) / ceil8(cols);
+  };
+  const bool x = fits(M, K), dy = fits(M, N), w = fits(N, K);
   if (x && w && ragged_pays(M, K)) r.products |= products & kFwd;
   if (dy && w && ragged_pays(M, N)) r.products |= products & kDgrad;
   if (x && dy) r.products |= products & kWgrad;

@@ -2427,9 +2427,10 @@ size_t gemm_fast_partial_bytes(int mode, int64_t I, int64_t J, int64_t R, int ke
 // 69.3 and 282 -> 278, 8192 x 1280 x 5120 114 -> 102 and 417 -> 408; two steps
 // lose, 8192 x 2560 x 1280 (67.5 -> 60.4 but 255 -> 260) and 8192 x 5120 x 1280
 // (134 -> 119 but 428 -> 437).  Below the rule's line the steps lose by 1 - 3%:
-// 4096 x 1280 x 1280, 4096 x 10240 x 1280, 16384 x 640 x 640.  Below 4e9 products the pass's fixed time takes the gain.  A split dgrad
-// keeps the packed kernel: the WGRAD launch carries its reduction
-// (2048 x 1280 x 5120: 42.8 -> 42 without that).
+// 4096 x 1280 x 1280, 4096 x 10240 x 1280, 16384 x 640 x 640.  Below 4e9
+// products the pass's fixed time takes the gain.  A split dgrad keeps the packed
+// kernel: the WGRAD launch carries its reduction (2048 x 1280 x 5120: 42.8 -> 42
+// without that).
 bool gemm_decode_pays(int mode, int64_t I, int64_t J, int64_t R) {
   if ((double)I * (double)J * (double)R < 4e9 || J % 8 != 0 || R % 8 != 0) return false;
   if (mode == MODE_FWD) return I >= 8192 && (double)I * (double)J * (double)R >= 1.6e10;

@@ -261,6 +261,7 @@ def test_calls_that_write_operands_get_a_workspace_of_their_own(L):
 @pytest.mark.parametrize("M,N,K,copied", [
     (16384, 50257, 768, 50264 * 768 * 2),            # dy's copy would pass 2^30 bytes: the weight's alone, for the forward
     (16384, 768, 50257, 768 * 50264 * 2),            # x's likewise: the weight's, for the dgrad
+    (1 << 20, 505, 8, (1 << 20) * 512 * 2 + 512 * 8 * 2),   # dy's copy ends 14 bytes short of them
     (16384, 65, 384, 16384 * 72 * 2 + 72 * 384 * 2),   # x has whole chunks
     (2048, 320, 36, 2048 * 40 * 2 + 320 * 40 * 2),     # dy has
     (4, 33, 31, 4 * 32 * 2 + 4 * 40 * 2),              # too few rows and terms for the forward and the dgrad
